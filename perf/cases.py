@@ -5,16 +5,17 @@ Kinds of case (`kind`):
            step that bench.py times): D2Z.run() -> zreion
   field    the step of a loop over realisations: hand over a new device field, run,
            read the per-radius table (R, sigma, sigma_grid) and zreion
-  driver   the d2z program's own flow on host arrays: ICs in, zreion and bubble
-           radii out (RecordBubbleSizes = 1)
+  driver   the d2z program's own flow on host arrays: ICs in, zreion out
   group    uneven boxes of one sweep stepped together (Group.run())
   history  the d2z program from its transform to the corrected output: run,
            GetHistory, bubble mean free paths, corrected history, remapped zreion
   power    binned power spectrum of a new device field
 
 Sizes are those of bench.py's workloads and of the tests; cells are about 1.5 to
-2 Mpc/h wide, as there.  Fields are Gaussian with a CDM-like spectrum.  At N =
-1024 the radii per batch are set so that several contexts fit one card.
+2 Mpc/h wide, as there.  Fields are Gaussian with a CDM-like spectrum.  Bubble
+radii (RecordBubbleSizes) are not among the outputs: the first radius that
+reaches a flat maximum is decided by rounding, so two right answers differ by
+whole radius steps.  At N = 1024 the radii per batch are set so that several contexts fit one card.
 """
 import math
 import sys
@@ -42,7 +43,7 @@ def listed():
         {"name": "field_64_fused", "kind": "field", "mode": "fused", "n": 64, "nscales": 8, "box": 100.0, "rmax": 25.0},
         # the 128^3 x 32 configuration: short kernels back to back
         {"name": "run_128_mixed", "kind": "run", "mode": "mixed", "n": 128, "nscales": 32, "box": 200.0, "rmax": 50.0},
-        # the d2z program on host data, a length with a factor 3, bubble radii recorded
+        # the d2z program on host data, a length with a factor 3
         {"name": "driver_192_fused", "kind": "driver", "mode": "fused", "n": 192, "nscales": 24, "box": 300.0,
          "rmax": 50.0},
         # the separate-kernel path in the reference's order
@@ -145,8 +146,7 @@ def _params(c, n, box):
     # at 1024^3 a batch of 16 FP32 radii (32 in FP16 storage) takes 69 GB of intermediates
     rpl = 16 if n == 1024 and c["mode"] != "half" else 0
     return prc_d2z.D2ZParams(N=n, Nscales=c["nscales"], BoxSize=box, Rmax=c["rmax"], zeta=ZETA, M_min=M_MIN,
-                             RecordBubbleSizes=int(c["kind"] == "driver"), mode=MODES[c["mode"]],
-                             radii_per_launch=rpl, **HOST_COSMOLOGY)
+                             mode=MODES[c["mode"]], radii_per_launch=rpl, **HOST_COSMOLOGY)
 
 
 def _context(c, n, box):
@@ -221,7 +221,7 @@ def run(state):
     if kind == "driver":
         d.set_delta(state["delta"])
         d.run()
-        return {"rbubble": d.rbubble(), "zreion": d.zreion()}
+        return {"zreion": d.zreion()}
     if kind == "power":
         d.set_delta_device(state["delta"].data_ptr())
         nk, kmin, kmax = state["bins"]
@@ -251,9 +251,7 @@ def work(case):
         return {k: sum(e[k] for e in each) for k in ("bytes", "flops")}
     w = step(case["n"], case["nscales"])
     m = float(case["n"]) ** 3
-    if kind == "driver":
-        w["bytes"] += 4.0 * m
-    elif kind == "history":  # the histogram's read and the remap's read and write, 4e7 skewers' cells
+    if kind == "history":  # the histogram's read and the remap's read and write, 4e7 skewers' cells
         w["bytes"] += 12.0 * m + 4.0 * 4e7
     elif kind == "power":
         w = {"bytes": 4.0 * m, "flops": 2.5 * m * math.log2(m) + 10.0 * m / 2}
@@ -348,7 +346,7 @@ def _inverse_erfc(y):
 
 
 def _exact_step(c, n, box, seed):
-    """zreion, the radius that set it and the per-radius table, from the field in FP64."""
+    """zreion and the per-radius table, from the field in FP64."""
     om, h, s8 = (float(np.float32(HOST_COSMOLOGY[k])) for k in ("Omegam", "h", "sigma8"))
     pn2 = s8 * s8 / _sigma2(8.0 / h)
     dens = 2.775e11 * om * h * h
@@ -365,7 +363,6 @@ def _exact_step(c, n, box, seed):
     # dk of the d2z program (float), |k| per plane of the spectrum
     dk = float(np.float32(2.0 * math.pi / float(np.float32(box) / np.float32(h))))
     zre = torch.zeros((n, n, n), device="cuda", dtype=torch.float64)
-    rb = torch.zeros_like(zre) if c["kind"] == "driver" else None
     grid = []
     # W by |k|^2 in units of dk^2, an integer
     m2 = (fx[:, None, None] ** 2 + fx[None, :, None] ** 2 + fz[None, None, :] ** 2).int()
@@ -383,13 +380,9 @@ def _exact_step(c, n, box, seed):
         if s2 > smin2:
             continue
         z = d.add_(math.sqrt(2 * (smin2 - s2)) * erfz).mul_(A).sub_(1.0)
-        if rb is not None:
-            rb[z > zre] = float(r)
         torch.maximum(zre, z, out=zre)
         del d, z
     out = {"zreion": zre}
-    if rb is not None:
-        out["rbubble"] = rb
     if grid:
         out["table"] = np.stack([R * h, np.sqrt(sig2), np.array(grid)], axis=1)
     return out
