@@ -405,16 +405,26 @@ struct FxLds {
   static constexpr int NROW = P::L + (P::L >> SH);  // padded exchange rows
   static constexpr int SMEM = NROW * CF;           // float2
   static constexpr int KTAB = (CF + 1) * (P::L / 2 + 1);  // float
+  // the plan's twiddles in LDS (float2); none at N = 2048, where they do not fit
+  // beside the largest W(x) table and are read from memory
+  static constexpr bool TW = P::L <= 1024;
+  static constexpr int NTW = TW ? (plan_tw_size<P>() > 0 ? plan_tw_size<P>() : 1) : 1;
 };
 
-// One tile (ky, kz block, column sub-tile) of the fused x pass for nb radii;
-// wsh (the W(x) table, wM intervals) must be in LDS before the call.
+// One tile (ky, kz block, column sub-tile) of the fused x pass for nb radii.
+// wsh (the W(x) table, wM intervals) and, with FxLds::TW, tw (the plan's
+// twiddles, transposed) are in LDS and may still be being written: the barrier
+// before the radius loop covers them.  The radius loop reads no global memory
+// but the packed lanes' DN: loads return in order behind the stores that a wave
+// issued before them, so twiddles read from memory made every radius wait for
+// the previous radius's stores (1024^3: 26.8 -> 24.2 ms per 16 radii; N <= 512
+// unchanged within 1%).
 template <class P, int C, int CF, class TS>
 __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const float2* __restrict__ D0,
                                         const float2* __restrict__ DN, TS* __restrict__ Tbuf, float dk, float invN3,
                                         const RadiusConst* __restrict__ rc, int r0, int nb,
-                                        const float2* __restrict__ tw, const float4* wsh, int wM, float winvh,
-                                        long long tile, float2* smem, float* ktab) {
+                                        const float2* tw, const float4* wsh, int wM, float winvh, long long tile,
+                                        float2* smem, float* ktab) {
   constexpr int N = P::L, T = P::T, E = P::E;
   constexpr int NSUB = C / CF;
   constexpr int NF = N / 2 + 1;           // distinct |fx|
@@ -485,7 +495,7 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
     }
     lds_hold(v);      // the table reads stay above the barrier
     __syncthreads();  // table reads done before the transform reuses the buffer
-    pencil_fft<P, +1, 0, LdsColPad<SH>, false, false>(v, i, tw, lds);
+    pencil_fft<P, +1, 0, LdsColPad<SH>, FxLds<P, CF>::TW, false>(v, i, tw, lds);
     TS* dst = tp + (long long)rl * plane;
 #pragma unroll
     for (int e = 0; e < E; ++e) st(dst, (long long)(i + e * T) * N * C, v[e]);
@@ -500,12 +510,15 @@ __global__ void __launch_bounds__(P::T* CF)
   __shared__ float2 smem[FxLds<P, CF>::SMEM];
   __shared__ float ktab[FxLds<P, CF>::KTAB];  // |k|/dk of the table entries, same order
   extern __shared__ float4 wsh[];              // W(x) interpolation table (wM intervals)
+  __shared__ float2 s_tw[FxLds<P, CF>::NTW];
   for (int q = threadIdx.x; q < wM; q += P::T * CF) wsh[q] = wcoef[q];
+  if constexpr (FxLds<P, CF>::TW) copy_twiddles_transposed<P>(s_tw, tw, threadIdx.x, P::T * CF);
   // FP32 outputs: consecutive lines over the XCDs; FP16: one range per XCD
   const long long tile = std::is_same<TS, float2>::value
                              ? line_tile(blockIdx.x, gridDim.x, line_group(C / CF, C * (int)sizeof(TS)))
                              : xcd_tile(blockIdx.x, gridDim.x);
-  fx_body<P, C, CF, TS>(S, D0, DN, Tbuf, dk, invN3, rc, r0, nb, tw, wsh, wM, winvh, tile, smem, ktab);
+  fx_body<P, C, CF, TS>(S, D0, DN, Tbuf, dk, invN3, rc, r0, nb, FxLds<P, CF>::TW ? s_tw : tw, wsh, wM, winvh, tile,
+                        smem, ktab);
 }
 
 // columns per fused-x block: keep the block at <= 512 threads
@@ -834,7 +847,8 @@ constexpr size_t mb_lds_n(MBPass pass) {
     case MBPass::kFwdX:
     case MBPass::kInvY: return sizeof(float2) * TilePlan<N>::L * Blk<N>::C;
     case MBPass::kFx:
-      return sizeof(float2) * FxLds<PF, FxCols<N>::CF>::SMEM + sizeof(float) * FxLds<PF, FxCols<N>::CF>::KTAB;
+      return sizeof(float2) * (FxLds<PF, FxCols<N>::CF>::SMEM + FxLds<PF, FxCols<N>::CF>::NTW) +
+             sizeof(float) * FxLds<PF, FxCols<N>::CF>::KTAB;
     case MBPass::kFz:
       return sizeof(float2) * (FzLds<PZ>::SMEM + FzLds<PZ>::NTW + PZ::L);
     default: return 0;
@@ -940,7 +954,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
   extern __shared__ float4 mb_lds4[];
   float4* wsh = mb_lds4;
   float2* smem = reinterpret_cast<float2*>(mb_lds4 + maxM);
-  float* ktab = reinterpret_cast<float*>(smem + FxLds<P, CF>::SMEM);
+  float2* s_tw = smem + FxLds<P, CF>::SMEM;
+  float* ktab = reinterpret_cast<float*>(s_tw + FxLds<P, CF>::NTW);
+  static_assert(FxLds<P, CF>::TW, "the multi-box x pass keeps its twiddles in LDS");
   int loaded = -1;
   for (long long k = 0;; ++k) {
     const long long t = mbox_item(k, nitems);
@@ -950,10 +966,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
     if (b != loaded) {
       __syncthreads();  // the previous box's table is no longer read
       for (int q = threadIdx.x; q < B.wM; q += 256) wsh[q] = B.wcoef[q];
+      copy_twiddles_transposed<P>(s_tw, B.st_fx, threadIdx.x, 256);
       loaded = b;
     }
     float2* T = B.T + (long long)toff * ((long long)N * N * (N / 2));
-    fx_body<P, C, CF, float2>(B.S, B.D0, B.DN, T, B.dk, B.invN3, B.rc, r0, nb, B.st_fx, wsh, B.wM, B.winvh,
+    fx_body<P, C, CF, float2>(B.S, B.D0, B.DN, T, B.dk, B.invN3, B.rc, r0, nb, s_tw, wsh, B.wM, B.winvh,
                               t - first[b], smem, ktab);
     __syncthreads();
   }
