@@ -22,6 +22,28 @@ struct Blk {
   static constexpr int C = (N == 16 || N == 2048) ? 8 : 16;
 };
 
+// Rows of the FP32 intermediates T [kz/C][x][y][kz%C] of N >= 512: row y of plane
+// x is stored at y ^ ((x mod SW) << SH), 64 or 128 rows (8 KB) being the unit that
+// moves, so consecutive x put the same y on different 8 KB of their 64 KB or
+// 128 KB planes.  The x pass writes one y of every x; without it those stores are
+// a power of two apart and fall on a part of the memory channels.  Store-only
+// kernels with its pattern at 1024^3: 64 B halves of lines 2.6 -> 4.1 TB/s, whole
+// lines 4.5 -> 5.7 (512^3: 4.4 -> 5.7).  Padding the planes by 8 KB instead gave
+// 3.5 and 5.6, but tiles off their 128 KB boundaries cost the y pass 4%.  A y
+// tile stays one contiguous block whose SW pieces are permuted, SW values of x
+// apart by a multiple of SW share their permutation, and any 64 rows from a
+// multiple of 64 on stay consecutive.  FP16 planes and smaller grids, which the
+// Infinity Cache holds in part, gained nothing from it.
+template <int N, class TS>
+struct TLay {
+  static constexpr bool kOn = N >= 512 && sizeof(TS) == 8;
+  static constexpr int SW = !kOn ? 1 : (N == 512 ? 8 : 16);
+  static constexpr int SH = !kOn ? 0 : (N == 2048 ? 7 : 6);
+  static __device__ __forceinline__ int swap(int x) { return (x & (SW - 1)) << SH; }
+  // stored row index of z row r = x N + y
+  static __device__ __forceinline__ long long row(long long r) { return kOn ? r ^ swap((int)(r / N)) : r; }
+};
+
 // (kx, ky, kz) of blocked index id of the spectrum S = [kz/C][ky][kx][kz%C]
 struct SIndex {
   int kx, ky, kz;

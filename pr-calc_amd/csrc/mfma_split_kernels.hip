@@ -234,7 +234,10 @@ __global__ void __launch_bounds__(kFxThreads)
   const float bs = ldexpf(1.0f, 10 - e2), ibs = ldexpf(1.0f, e2 - 10);
   const float wscale = invN3 * bs;
 
-  float2* tp = Tbuf + (long long)kzb * kN * kN * kC + (long long)ky * kC + sub * kCF + c;
+  // all rows x of a wave have x mod 16 = w: one row permutation per wave
+  static_assert(TLay<kN, float2>::SW == 16, "x mod 16 is the wave index");
+  const int kyt = ky ^ TLay<kN, float2>::swap(w);
+  float2* tp = Tbuf + (long long)kzb * kN * kN * kC + (long long)kyt * kC + sub * kCF + c;
 
 #pragma unroll 1
   for (int rl = 0; rl < nb; ++rl) {
@@ -414,7 +417,7 @@ __global__ void __launch_bounds__(kFzThreads) __attribute__((amdgpu_waves_per_eu
   float2 pf[8];
   const long long lane_off = ((long long)lkzb * nrows + lrow) * 16 + lkz;
   auto fetch = [&](long long gbase, int q) {
-    const float2* tp = Tbuf + (long long)q * plane + gbase * 16 + lane_off;
+    const float2* tp = Tbuf + (long long)q * plane + TLay<kN, float2>::row(gbase) * 16 + lane_off;
 #pragma unroll
     for (int e = 0; e < 8; ++e) pf[e] = tp[(long long)(4 * e) * nrows * 16];
   };

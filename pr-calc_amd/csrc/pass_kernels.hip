@@ -3,7 +3,7 @@
 // Layouts (complex elements, C = Blk<N>::C, Nh = N/2, blocked as described in
 // d2z_device.h):
 //   S   spectrum      [kz/C][ky][kx][kz%C]   written once by the forward passes
-//   T_r intermediate  [kz/C][x][y][kz%C]     one per radius of a batch
+//   T_r intermediate  [kz/C][x][y][kz%C]     one per radius of a batch; rows y permuted (TLay)
 //   real fields       dense [x][y][z]
 // The kz = 0 slot of every row holds the packed pair H(kz=0) + i H(kz=N/2) of
 // the z transform (both real along z); the true planes kz = 0 and kz = N/2 of
@@ -35,7 +35,7 @@ __device__ __forceinline__ float2 ld(const __half2* p, long long i) { return __h
 __device__ __forceinline__ void st(float2* p, long long i, float2 v) { p[i] = v; }
 __device__ __forceinline__ void st(__half2* p, long long i, float2 v) { p[i] = __float22half2_rn(v); }
 
-// Offset of element k = i + e*T of z row r in the T layout ([k/C][rows][k%C]).
+// Offset of element k = i + e*T of stored z row r (TLay::row) in the T layout ([k/C][rows][k%C]).
 // When C divides T the offset advances by a constant per e.
 template <class P, int C>
 __device__ __forceinline__ long long zrow_offset(int i, int e, long long r, long long nrows) {
@@ -124,7 +124,7 @@ __device__ __forceinline__ void fwd_z_rows(const float* __restrict__ in, float2*
   r2c_post<P>(v, m, i, tw_full);
   if (valid) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[zrow_offset<P, C>(i, e, row, nrows)] = v[e];
+    for (int e = 0; e < E; ++e) out[zrow_offset<P, C>(i, e, TLay<2 * L, float2>::row(row), nrows)] = v[e];
   }
 }
 
@@ -141,33 +141,41 @@ __global__ void __launch_bounds__(256) k_fwd_z(const float* __restrict__ in, flo
 // Tile t -> (o, cb) = (t mod nOuter, t / nOuter); element (a, c) is read at
 // cb*sCB + o*in_sO + a*in_sA + c and written at cb*sCB + o*out_sO + a*out_sA + c
 // (in place when in == out with equal strides).
-template <class P, int C, int DIR, class TI, class TO>
+// The T layout's row permutation (TLay): along y (kYInPlace, outer index x) the
+// T strides of a thread's elements are permuted, element e at (e ^ x mod SW); an x
+// pass on its T side permutes the outer index ky by the thread's x = i + e*T,
+// the same for all e.
+template <class P, int C, int DIR, class TI, class TO, Axis AX>
 __device__ __forceinline__ void tile_body(const TI* in, TO* out, long long in_sA, long long in_sO, long long out_sA,
                                           long long out_sO, long long sCB, int nOuter, float oscale,
                                           const float2* __restrict__ tw, long long tile, float2* smem) {
   constexpr int T = P::T, E = P::E;
+  using TL = TLay<P::L, TI>;
+  static_assert(!TL::kOn || ((1 << TL::SH) == T && E % TL::SW == 0 && T % TL::SW == 0), "row permutation of the tile plan");
   const int tid = threadIdx.x;
   const int c = tid % C, i = tid / C;
   const long long o = tile % nOuter, cb = tile / nOuter;
-  // running pointers: element i + e*T sits e*T*sA after element i
-  const TI* ip = in + cb * sCB + o * in_sO + c + (long long)i * in_sA;
-  TO* op = out + cb * sCB + o * out_sO + c + (long long)i * out_sA;
+  const long long io = AX == Axis::kXTtoS ? o ^ TL::swap(i) : o, oo = AX == Axis::kXStoT ? o ^ TL::swap(i) : o;
+  const int perm = AX == Axis::kYInPlace ? (int)o & (TL::SW - 1) : 0;
+  // element i + e*T sits e*T*sA after element i
+  const TI* ip = in + cb * sCB + io * in_sO + c + (long long)i * in_sA;
+  TO* op = out + cb * sCB + oo * out_sO + c + (long long)i * out_sA;
   const long long istep = (long long)T * in_sA, ostep = (long long)T * out_sA;
   float2 v[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e, ip += istep) v[e] = ld(ip, 0);
+  for (int e = 0; e < E; ++e) v[e] = ld(ip, (e ^ perm) * istep);
   pencil_fft<P, DIR>(v, i, tw, LdsPencil{smem + c, C});
 #pragma unroll
-  for (int e = 0; e < E; ++e, op += ostep) st(op, 0, cscale(v[e], oscale));
+  for (int e = 0; e < E; ++e) st(op, (e ^ perm) * ostep, cscale(v[e], oscale));
 }
 
-template <class P, int C, int DIR, class TI, class TO>
+template <class P, int C, int DIR, class TI, class TO, Axis AX>
 __global__ void __launch_bounds__(P::T* C)
     k_tile(const TI* in, TO* out, long long in_sA, long long in_sO, long long out_sA, long long out_sO,
            long long sCB, int nOuter, float oscale, const float2* __restrict__ tw) {
   __shared__ float2 smem[P::L * C];
-  tile_body<P, C, DIR, TI, TO>(in, out, in_sA, in_sO, out_sA, out_sO, sCB, nOuter, oscale, tw,
-                               xcd_tile(blockIdx.x, gridDim.x), smem);
+  tile_body<P, C, DIR, TI, TO, AX>(in, out, in_sA, in_sO, out_sA, out_sO, sCB, nOuter, oscale, tw,
+                                   xcd_tile(blockIdx.x, gridDim.x), smem);
 }
 
 // Persistent in-place tile pass (the y passes; TS = float2 or __half2 storage):
@@ -190,15 +198,18 @@ __global__ void __launch_bounds__(P::T* C)
   __syncthreads();
   const long long istep = (long long)T * sA;
   const long long lane_off = c + (long long)i * sA;
-  auto tile_base = [&](long long vb) {
+  using TL = TLay<L, TS>;
+  auto tile_base = [&](long long vb, int& perm) {
     const long long tile = xcd_tile(vb, ntiles);
+    perm = (int)(tile % nOuter) & (TL::SW - 1);  // the plane's row permutation: see tile_body
     return (tile / nOuter) * sCB + (tile % nOuter) * sO + lane_off;
   };
   TS raw[E];
   auto fetch = [&](long long vb) {
-    const TS* p = data + tile_base(vb);
+    int perm;
+    const TS* p = data + tile_base(vb, perm);
 #pragma unroll
-    for (int e = 0; e < E; ++e) raw[e] = p[e * istep];
+    for (int e = 0; e < E; ++e) raw[e] = p[(e ^ perm) * istep];
   };
   long long vb = blockIdx.x;
   if (vb < ntiles) fetch(vb);
@@ -209,9 +220,10 @@ __global__ void __launch_bounds__(P::T* C)
     for (int e = 0; e < E; ++e) v[e] = ld(raw + e, 0);
     if (vb + gridDim.x < ntiles) fetch(vb + gridDim.x);
     pencil_fft<P, DIR, 0, LdsPencil, false, false>(v, i, s_tw, LdsPencil{smem + c, C});
-    TS* op = data + tile_base(vb);
+    int perm;
+    TS* op = data + tile_base(vb, perm);
 #pragma unroll
-    for (int e = 0; e < E; ++e) st(op, e * istep, cscale(v[e], oscale));
+    for (int e = 0; e < E; ++e) st(op, (e ^ perm) * istep, cscale(v[e], oscale));
   }
 }
 
@@ -228,7 +240,7 @@ __global__ void __launch_bounds__(256) k_inv_z(const TS* __restrict__ in, float*
   const int i = t % T, rr = t / T;
   const long long row = (long long)blockIdx.x * ROWS + rr;
   const bool valid = row < nrows;
-  const long long r = valid ? row : 0;
+  const long long r = TLay<2 * L, TS>::row(valid ? row : 0);
   float2 v[E], m[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) v[e] = ld(in, zrow_offset<P, C>(i, e, r, nrows));
@@ -455,7 +467,9 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
     m[e] = packed ? D0[(long long)kx * N + ky] : sp[(long long)kx * C];
   }
   const int fy2 = fsq(ky, N);
-  TS* tp = Tbuf + (long long)kzb * N * N * C + (long long)ky * C + sub * CF + cl;  // element x at tp[x*N*C]
+  static_assert(T % TLay<N, TS>::SW == 0, "x = i + e*T permutes its rows by i");
+  const int kyt = ky ^ TLay<N, TS>::swap(i);  // stored row of ky in the planes of this thread's x
+  TS* tp = Tbuf + (long long)kzb * N * N * C + (long long)kyt * C + sub * CF + cl;  // element x at tp[x*N*C]
   const LdsColPad<SH> lds{smem + cl, CF};
   const int ntab = (has_packed ? CF + 1 : CF) * NF;
   for (int q = tid; q < ntab; q += NT) {
@@ -541,14 +555,18 @@ struct FxPlan<2048> {
 };
 
 // Columns per fused x block: at most 512 threads, except with the 8-element
-// plans, which take 1024 threads: 8 columns x 128 at N = 1024 (64 B segments
-// per row; 4 columns, 32 B segments, made the FP32 stores far slower) and
-// 4 columns x 256 at N = 2048 (C = 8 there).
+// plans, which take 1024 threads: 16 columns x 64 at N = 512 (whole 128 B lines
+// per row in FP32: 10.6 -> 8.35 ms per 512^3 x 64 step against two 512-thread
+// blocks of 8 columns per CU, FP16 9.5 -> 8.1), 8 columns x 128 at N = 1024
+// (64 B segments per row; 4 columns, 32 B segments, made the FP32 stores far
+// slower, and 16 do not fit the LDS) and 4 columns x 256 at N = 2048 (C = 8
+// there).
 template <int N>
 struct FxCols {
   using P = typename FxPlan<N>::P;
   static constexpr int C = Blk<N>::C;
   static constexpr int CF = (N == 1024)   ? 8
+                            : (N == 512)  ? 16
                             : (N == 2048) ? 4
                                           : ((P::T * C <= 512) ? C : (P::T * (C / 2) <= 512 ? C / 2 : C / 4));
 };
@@ -619,7 +637,7 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
   const double sc = (double)iscale, sc2 = sc * sc;
   const long long row = base + rr;
   const bool valid = row < nrows;
-  const long long r = valid ? row : 0;
+  const long long r = TLay<2 * L, TS>::row(valid ? row : 0);
   float2 best[E];
   float bR0[E], bR1[E];
 #pragma unroll
@@ -913,8 +931,9 @@ __global__ void __launch_bounds__(256) k_mb_tile(const MBox* __restrict__ boxes,
       const TileMap m = mb_tile_map<N>(pass, nb);
       const float2* in = B.T;
       float2* out = (pass == MBPass::kFwdX) ? B.S : B.T;
-      tile_body<P, Blk<N>::C, DIR, float2, float2>(in, out, m.in_sA, m.in_sO, m.out_sA, m.out_sO, m.sCB, m.nOuter,
-                                                   1.0f, B.st_full, item, smem);
+      static_assert(!TLay<N, float2>::kOn, "multi-box planes are stored in row order");
+      tile_body<P, Blk<N>::C, DIR, float2, float2, Axis::kYInPlace>(in, out, m.in_sA, m.in_sO, m.out_sA, m.out_sO,
+                                                                    m.sCB, m.nOuter, 1.0f, B.st_full, item, smem);
     });
     __syncthreads();
   }
@@ -1254,15 +1273,24 @@ static hipError_t inv_z_impl(const TS* in, float* out, float iscale, const float
   return hipGetLastError();
 }
 
-template <int N, int DIR, class TI, class TO>
-static hipError_t tile_impl(const TI* in, TO* out, const TileMap& mp, float oscale, const float2* tw,
-                            hipStream_t s) {
+template <int N, int DIR, class TI, class TO, Axis AX>
+static hipError_t tile_axis(const TI* in, TO* out, const TileMap& mp, float oscale, const float2* tw, hipStream_t s) {
   using P = TilePlan<N>;
   constexpr int C = Blk<N>::C;
   const long long ntiles = (long long)mp.nOuter * mp.nColBlocks;
-  hipLaunchKernelGGL((k_tile<P, C, DIR, TI, TO>), dim3((unsigned)ntiles), dim3(P::T * C), 0, s, in, out, mp.in_sA,
+  hipLaunchKernelGGL((k_tile<P, C, DIR, TI, TO, AX>), dim3((unsigned)ntiles), dim3(P::T * C), 0, s, in, out, mp.in_sA,
                      mp.in_sO, mp.out_sA, mp.out_sO, mp.sCB, mp.nOuter, oscale, tw);
   return hipGetLastError();
+}
+
+template <int N, int DIR, class TI, class TO>
+static hipError_t tile_impl(const TI* in, TO* out, const TileMap& mp, float oscale, const float2* tw,
+                            hipStream_t s) {
+  if constexpr (TLay<N, TI>::kOn) {  // the axis decides where rows are permuted
+    if (mp.axis == Axis::kXTtoS) return tile_axis<N, DIR, TI, TO, Axis::kXTtoS>(in, out, mp, oscale, tw, s);
+    if (mp.axis == Axis::kXStoT) return tile_axis<N, DIR, TI, TO, Axis::kXStoT>(in, out, mp, oscale, tw, s);
+  }
+  return tile_axis<N, DIR, TI, TO, Axis::kYInPlace>(in, out, mp, oscale, tw, s);
 }
 
 // Blocks of kernel f (threads per block) resident on the current device at once
@@ -1410,6 +1438,7 @@ TileMap tile_map(int N, Axis axis) {
   m.nOuter = N;
   m.nColBlocks = (N / 2) / C;
   m.sCB = (long long)N * N * C;
+  m.axis = axis;
   switch (axis) {
     case Axis::kYInPlace:  // T layout (x, y): tile (x, kz block), transform along y
       m.in_sA = m.out_sA = C;
