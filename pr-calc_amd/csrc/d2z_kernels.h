@@ -55,6 +55,14 @@ struct GrfSpectrum {
 constexpr int kFusedMaxRadii = 32;  // radii per fused batch (y and z passes)
 constexpr int kFxMaxRadii = 16;     // radii per x-pass launch (a batch takes one or more)
 
+// Strides of one tiled pass (complex elements); see pass_kernels.hip.
+enum class Axis { kYInPlace, kXTtoS, kXStoT };
+struct TileMap {
+  long long in_sA, in_sO, out_sA, out_sO, sCB;
+  int nOuter, nColBlocks;
+  Axis axis;
+};
+
 // Cubic Hermite table of the top-hat window W(x) = 3 (sin x - x cos x) / x^3 on
 // [0, M h): interval i holds (c0, c1, c2, c3) with W(x_i + t h) = c0 + t (c1 +
 // t (c2 + t c3)), built from W and W' in FP64 at the nodes.  M = 0: no table
