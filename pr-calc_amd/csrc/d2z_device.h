@@ -204,6 +204,17 @@ __host__ __device__ inline double barrier_offset(float dd, float erfizeta) {
   return sqrt(2. * (double)dd) * (double)erfizeta;
 }
 
+// q = ((double)z - 49.9) / dz, the history bin before truncation, with the same
+// integer part: a product by 1/dz (rdz) is within 3e-11 of the quotient for any
+// q of the table's range, so only values near an integer (about 2e-7 of all) take
+// the division, which costs some thirty FP64 instructions.
+__device__ __forceinline__ double history_q(float z, double dz, double rdz) {
+  const double d = (double)z - 49.9;
+  double q = d * rdz;
+  if (fabs(q - rint(q)) < 1e-7) q = d / dz;
+  return q;
+}
+
 // -------------------------------------- barrier: d2z() in double, stored float
 // z = A*(delta_R + B) - 1 with A float and B = sqrt(2 (smin^2 - s^2)) * erfizeta
 // in double (delta2zreion_d2z.C:206-216); separate multiply and subtract (no

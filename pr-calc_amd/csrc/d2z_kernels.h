@@ -206,9 +206,11 @@ hipError_t launch_moments_finish(const double2* partial, int nblk, int nrad, dou
 hipError_t launch_history(const float* zre, long long total, unsigned int* counts, double dz, int* range,
                           hipStream_t s);
 // history correction (bubble_kernels.hip)
-hipError_t launch_skewers(const float* zre, const float* zcur, const SkewerParams& p, double* sums,
+// scratch: N^3 floats and N + 1 doubles, 8-byte aligned
+hipError_t launch_skewers(const float* zre, const float* zcur, const SkewerParams& p, void* scratch, double* sums,
                           unsigned int* counts, int* fail, hipStream_t s);
-hipError_t launch_zvz(const float* history, const float* chist, float dzch, float* zvz, hipStream_t s);
+// rising: chist[q] <= chist[q + 1] for all q
+hipError_t launch_zvz(const float* history, const float* chist, float dzch, bool rising, float* zvz, hipStream_t s);
 hipError_t launch_remap(float* zre, long long n, const float* zvz, double dz, hipStream_t s);
 hipError_t launch_setup(const SetupParams& p, double* integ, float* Rr, double* Rint, SetupScalars* sc,
                         RadiusConst* rc, float* sigma_out, hipStream_t s);

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
+#include <string.h>
 
 #include "d2z_device.h"
 #include "d2z_kernels.h"
@@ -107,56 +108,75 @@ __global__ void k_maxabs(const float* __restrict__ x, long long n, unsigned int*
 
 // ------------------------------------------------ history histogram (GPU)
 // bin = (int)((z - 49.9)/dzhistory) in double (bubblehistory_d2z.C:17-28);
-// integer counts.  A first pass finds the lowest and highest occupied bin; then
-// block (chunk, w) counts the bins of window [lo + w W, lo + (w + 1) W) in an LDS
-// histogram (LDS atomics) and adds its non-zero bins to the global counts.
+// integer counts.  A first pass finds the lowest and highest occupied bin: the
+// bin does not increase with z, so these are the bins of the largest and smallest
+// z in the table's range [zmin, zmax], and only those two per block are divided.
+// Then block (chunk, w) counts the bins of window [lo + w W, lo + (w + 1) W) in
+// an LDS histogram (LDS atomics) and adds its non-zero bins to the global counts.
 // Windows past the highest bin return at once, so a field whose bins span
 // fewer than W (the usual case: zreion between ~5 and ~20 spans ~30000) is read
 // twice in all.
 constexpr int kHistWindow = 36000;  // bins per window: 144 KB of LDS
 constexpr int kHistWindows = (kNHistory + kHistWindow - 1) / kHistWindow;
 
-__device__ __forceinline__ int history_bin(float z, double dz) {
-  const double q = ((double)z - 49.9) / dz;
+__device__ __forceinline__ int history_bin(float z, double dz, double rdz) {
+  const double q = history_q(z, dz, rdz);
   return (q > -1.0 && q < (double)kNHistory) ? (int)q : -1;  // NaN: -1
 }
 
-__global__ void __launch_bounds__(256) k_history_range(const float* __restrict__ zre, long long total,
-                                                       int* __restrict__ range, double dz) {
-  int lo = kNHistory, hi = -1;
+// One pair of atomics per block, and only where it moves the range: 2048 blocks
+// with a pair per wave queued 16384 of them on two addresses (192 us at 256^3).
+__global__ void __launch_bounds__(1024) k_history_range(const float* __restrict__ zre, long long total,
+                                                        int* __restrict__ range, double dz, float zmin, float zmax) {
+  float mn = INFINITY, mx = -INFINITY;  // smallest and largest z in [zmin, zmax]
+  auto take = [&](float z) {
+    const bool in = z >= zmin && z <= zmax;
+    mn = fminf(mn, in ? z : INFINITY);
+    mx = fmaxf(mx, in ? z : -INFINITY);
+  };
   const long long n4 = total >> 2;
   const float4* z4 = reinterpret_cast<const float4*>(zre);
   const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n4; id += stride) {
-    const float4 v = z4[id];
-    const int b[4] = {history_bin(v.x, dz), history_bin(v.y, dz), history_bin(v.z, dz), history_bin(v.w, dz)};
+  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n4; id += 4 * stride) {
+    float4 v[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (b[q] >= 0) {
-        lo = min(lo, b[q]);
-        hi = max(hi, b[q]);
-      }
-  }
-  for (long long id = 4 * n4 + (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total; id += stride) {
-    const int b = history_bin(zre[id], dz);
-    if (b >= 0) {
-      lo = min(lo, b);
-      hi = max(hi, b);
+    for (int u = 0; u < 4; ++u) v[u] = z4[id + u * stride < n4 ? id + u * stride : id];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      take(v[u].x);
+      take(v[u].y);
+      take(v[u].z);
+      take(v[u].w);
     }
   }
+  for (long long id = 4 * n4 + (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total; id += stride) take(zre[id]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    lo = min(lo, __shfl_xor(lo, off, 64));
-    hi = max(hi, __shfl_xor(hi, off, 64));
+    mn = fminf(mn, __shfl_xor(mn, off, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
   }
-  if ((threadIdx.x & 63) == 0 && hi >= 0) {
-    atomicMin(&range[0], lo);
-    atomicMax(&range[1], hi);
+  __shared__ float s_mn[16], s_mx[16];
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    s_mn[w] = mn;
+    s_mx[w] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) {
+      mn = fminf(mn, s_mn[k]);
+      mx = fmaxf(mx, s_mx[k]);
+    }
+    if (mn <= mx) {
+      const int lo = (int)(((double)mx - 49.9) / dz), hi = (int)(((double)mn - 49.9) / dz);
+      if (lo < __hip_atomic_load(&range[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&range[0], lo);
+      if (hi > __hip_atomic_load(&range[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&range[1], hi);
+    }
   }
 }
 
 __global__ void __launch_bounds__(1024) k_history(const float* __restrict__ zre, long long total,
-                                                  unsigned int* __restrict__ counts, double dz,
+                                                  unsigned int* __restrict__ counts, double dz, double rdz,
                                                   const int* __restrict__ range) {
   __shared__ unsigned int h[kHistWindow];
   if (range[1] < 0) return;  // no cell in any bin
@@ -170,16 +190,15 @@ __global__ void __launch_bounds__(1024) k_history(const float* __restrict__ zre,
   for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n4; id += 2 * stride) {
     const float4 v = z4[id];
     const float4 u = id + stride < n4 ? z4[id + stride] : make_float4(NAN, NAN, NAN, NAN);
-    const int b[8] = {history_bin(v.x, dz), history_bin(v.y, dz), history_bin(v.z, dz), history_bin(v.w, dz),
-                      history_bin(u.x, dz), history_bin(u.y, dz), history_bin(u.z, dz), history_bin(u.w, dz)};
+    const float z[8] = {v.x, v.y, v.z, v.w, u.x, u.y, u.z, u.w};
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int r = b[q] - lo;
-      if (b[q] >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
+      const int b = history_bin(z[q], dz, rdz), r = b - lo;
+      if (b >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
     }
   }
   for (long long id = 4 * n4 + (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total; id += stride) {
-    const int b = history_bin(zre[id], dz), r = b - lo;
+    const int b = history_bin(zre[id], dz, rdz), r = b - lo;
     if (b >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
   }
   __syncthreads();
@@ -479,21 +498,49 @@ hipError_t launch_moments_finish(const double2* partial, int nblk, int nrad, dou
   return hipGetLastError();
 }
 
+// largest float whose history bin ((double)z - 49.9)/dz (dz < 0) satisfies ok,
+// which holds at z = a and fails at z = b (a < b positive or zero), or smallest
+// where it fails at a and holds at b
+template <class F>
+static float history_edge(float a, float b, F ok) {
+  uint32_t ia, ib;
+  memcpy(&ia, &a, 4);
+  memcpy(&ib, &b, 4);
+  const bool first = ok(a);
+  while (ib - ia > 1) {
+    const uint32_t im = ia + (ib - ia) / 2;
+    float m;
+    memcpy(&m, &im, 4);
+    if (ok(m) == first) ia = im;
+    else ib = im;
+  }
+  const uint32_t r = first ? ia : ib;
+  float z;
+  memcpy(&z, &r, 4);
+  return z;
+}
+
 hipError_t launch_history(const float* zre, long long total, unsigned int* counts, double dz, int* range,
                           hipStream_t s) {
   // range = {0x7f7f7f7f (above every bin), -1} before the min/max pass
   hipError_t e = hipMemsetAsync(range, 0x7f, sizeof(int), s);
   if (e == hipSuccess) e = hipMemsetAsync(range + 1, 0xff, sizeof(int), s);
   if (e != hipSuccess) return e;
-  long long g = (total / 4 + 255) / 256;
-  if (g > 2048) g = 2048;
+  // the z that have a bin: q > -1 bounds them above (z < 49.9 + |dz|), q < NHISTORY below
+  const float zmax = history_edge(1.0f, 100.0f, [&](float z) { return ((double)z - 49.9) / dz > -1.0; });
+  const float zmin = history_edge(0.0f, 1.0f, [&](float z) { return ((double)z - 49.9) / dz < (double)kNHistory; });
+  // at least 16 loads of 16 B per thread, two blocks per CU at most
+  long long g = (total / 4 + 16 * 1024 - 1) / (16 * 1024);
+  if (g > 512) g = 512;
   if (g < 1) g = 1;
-  hipLaunchKernelGGL(k_history_range, dim3((unsigned)g), dim3(256), 0, s, zre, total, range, dz);
+  hipLaunchKernelGGL(k_history_range, dim3((unsigned)g), dim3(1024), 0, s, zre, total, range, dz, zmin, zmax);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  long long gh = (total / 8 + 1023) / 1024;
+  // a block adds up to ~30000 bins to the global counts: give it 2^18 cells for them
+  long long gh = (total + (1 << 18) - 1) >> 18;
   if (gh > 256) gh = 256;
   if (gh < 1) gh = 1;
-  hipLaunchKernelGGL(k_history, dim3((unsigned)gh, kHistWindows), dim3(1024), 0, s, zre, total, counts, dz, range);
+  hipLaunchKernelGGL(k_history, dim3((unsigned)gh, kHistWindows), dim3(1024), 0, s, zre, total, counts, dz, 1.0 / dz,
+                     range);
   return hipGetLastError();
 }
 

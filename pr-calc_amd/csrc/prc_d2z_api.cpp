@@ -1100,7 +1100,8 @@ int prc_d2z_bubble_mfp(prc_d2z_ctx* c, const float* history, int nskewers, uint6
   PRC_CHECK(c, hipMemsetAsync(c->d_mfp_sum, 0, sizeof(double) * kNXMfp, s), "skewers");
   PRC_CHECK(c, hipMemsetAsync(c->d_mfp_cnt, 0, sizeof(unsigned) * kNXMfp * kNMfp, s), "skewers");
   PRC_CHECK(c, hipMemsetAsync(c->d_flag, 0, sizeof(int), s), "skewers");
-  PRC_CHECK(c, launch_skewers(c->d_zre, c->d_zcur, sp, c->d_mfp_sum, c->d_mfp_cnt, c->d_flag, s), "skewers");
+  // the intermediates are free between runs: at least N^3 complex
+  PRC_CHECK(c, launch_skewers(c->d_zre, c->d_zcur, sp, c->d_T, c->d_mfp_sum, c->d_mfp_cnt, c->d_flag, s), "skewers");
   std::vector<double> sums(kNXMfp);
   std::vector<unsigned> cnt((size_t)kNXMfp * kNMfp);
   int failed = 0;
@@ -1155,7 +1156,9 @@ int prc_d2z_correct_zreion(prc_d2z_ctx* c, const float* history, const float* ch
   PRC_CHECK(c, hipMemcpyAsync(c->d_hin, history, sizeof(float) * kNHistory, hipMemcpyHostToDevice, s), "correct");
   PRC_CHECK(c, hipMemcpyAsync(c->d_chist, chistory, sizeof(float) * kNCHistory, hipMemcpyHostToDevice, s),
             "correct");
-  PRC_CHECK(c, launch_zvz(c->d_hin, c->d_chist, chistory_dz(), c->d_zvz, s), "correct");
+  bool rising = true;
+  for (int i = 0; i + 1 < kNCHistory; ++i) rising &= chistory[i] <= chistory[i + 1];
+  PRC_CHECK(c, launch_zvz(c->d_hin, c->d_chist, chistory_dz(), rising, c->d_zvz, s), "correct");
   PRC_CHECK(c, hipMemcpyAsync(zvz.data(), c->d_zvz, sizeof(float) * kNHistory, hipMemcpyDeviceToHost, s), "correct");
   PRC_CHECK(c, hipStreamSynchronize(s), "correct");
   // bins without a value take the next bin's (CorrectHistory, :316)
