@@ -215,9 +215,16 @@ hipError_t launch_remap(float* zre, long long n, const float* zvz, double dz, hi
 hipError_t launch_setup(const SetupParams& p, double* integ, float* Rr, double* Rint, SetupScalars* sc,
                         RadiusConst* rc, float* sigma_out, hipStream_t s);
 
-hipError_t launch_count_nonfinite(const float* x, long long n, int* flag, hipStream_t s);
-// *out = bits of max |x| (not for graph capture: clears with a memset)
-hipError_t launch_maxabs(const float* x, long long n, unsigned int* out, hipStream_t s);
+// one pass over an input field of `rows` rows of `width` floats, `stride` apart:
+// copied to dst (nullptr: read only; dst rows back to back) and checked; out
+// (host memory that the device can write) gets one entry per block
+struct FieldCheck {
+  unsigned int maxbits;  // max |x| of the block's cells as float bits; >= 0x7f800000: a NaN or Inf
+};
+constexpr int kFieldChecks = 2048;
+int take_field_blocks(long long n);
+hipError_t launch_take_field(const float* src, long long stride, float* dst, int width, long long rows,
+                             FieldCheck* out, hipStream_t s);
 hipError_t launch_fill(float* p, long long n, float v, hipStream_t s);
 hipError_t launch_sigma_finish(const double* partial, int nblk, int nrad, double invN3, float* sigma_grid_out,
                                hipStream_t s);

@@ -85,25 +85,48 @@ __global__ void k_moments_finish(const double2* __restrict__ partial, int nblk, 
   if (threadIdx.x == 0) sigma_grid_out[r0 + r] = (float)sqrt(a * invN3);
 }
 
-// ------------------------------------------------ input check
-// flag = 1 if any cell is NaN or Inf (plain vector stores of the same value).
-__global__ void k_nonfinite(const float* __restrict__ x, long long n, int* __restrict__ flag) {
-  int bad = 0;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n;
-       id += (long long)gridDim.x * blockDim.x)
-    bad |= !isfinite(x[id]);
-  if (bad) *flag = 1;
-}
-
-// max |x| as the bit pattern of a non-negative float (ordered as unsigned)
-__global__ void k_maxabs(const float* __restrict__ x, long long n, unsigned int* __restrict__ out) {
-  float m = 0.0f;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n;
-       id += (long long)gridDim.x * blockDim.x)
-    m = fmaxf(m, fabsf(x[id]));
+// ------------------------------------------------ input field
+// One pass over a field [rows][width]: copies it to dst (rows back to back;
+// dst = nullptr: no copy), and per block whether a cell is NaN or Inf and the
+// largest |x| as the bit pattern of a non-negative float.  The blocks' results go
+// to out[block], in host memory that the kernel writes directly, so nothing is
+// cleared before and copied back after.  V: float4 where source, destination
+// and rows allow it.
+template <class V>
+__global__ void __launch_bounds__(256) k_take_field(const float* __restrict__ src, long long stride, float* __restrict__ dst,
+                                                    int width, long long rows, FieldCheck* __restrict__ out) {
+  constexpr int W = sizeof(V) / sizeof(float);
+  const int wv = width / W;
+  const long long n = rows * wv, step = (long long)gridDim.x * 256;
+  const bool dense = stride == width;
+  unsigned int mx = 0u;  // |x| bits: Inf and NaN are >= 0x7f800000
+  auto at = [&](long long id) {
+    return reinterpret_cast<const V*>(dense ? src + id * W : src + id / wv * stride + id % wv * W);
+  };
+  auto take = [&](float x) { mx = max(mx, __float_as_uint(x) & 0x7fffffffu); };
+  for (long long id = (long long)blockIdx.x * 256 + threadIdx.x; id < n; id += 4 * step) {
+    V v[4];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));
+    for (int u = 0; u < 4; ++u) v[u] = *at(id + u * step < n ? id + u * step : id);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (W == 4) {
+        take(v[u].x);
+        take(v[u].y);
+        take(v[u].z);
+        take(v[u].w);
+      } else {
+        take(v[u]);
+      }
+      if (dst && id + u * step < n) reinterpret_cast<V*>(dst)[id + u * step] = v[u];
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = max(mx, (unsigned int)__shfl_xor((int)mx, off, 64));
+  __shared__ unsigned int s[4];
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x].maxbits = max(max(s[0], s[1]), max(s[2], s[3]));
 }
 
 // ------------------------------------------------ history histogram (GPU)
@@ -616,17 +639,21 @@ hipError_t launch_wtable(float4* coef, int M, double h, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_maxabs(const float* x, long long n, unsigned int* out, hipStream_t s) {
-  hipError_t e = hipMemsetAsync(out, 0, sizeof(unsigned int), s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_maxabs, dim3(grid1(n, 256, 8192)), dim3(256), 0, s, x, n, out);
-  return hipGetLastError();
+int take_field_blocks(long long n) {
+  // 16 loads of 16 B per thread, at most 8 blocks per CU
+  long long g = (n / 4 + 16 * 256 - 1) / (16 * 256);
+  return (int)(g < 1 ? 1 : (g > kFieldChecks ? kFieldChecks : g));
 }
 
-hipError_t launch_count_nonfinite(const float* x, long long n, int* flag, hipStream_t s) {
-  hipError_t e = hipMemsetAsync(flag, 0, sizeof(int), s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_nonfinite, dim3(grid1(n, 256, 8192)), dim3(256), 0, s, x, n, flag);
+hipError_t launch_take_field(const float* src, long long stride, float* dst, int width, long long rows,
+                             FieldCheck* out, hipStream_t s) {
+  const dim3 g(take_field_blocks(rows * width));
+  const bool vec = (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) % 16 == 0 && stride % 4 == 0 &&
+                   width % 4 == 0;
+  if (vec)
+    hipLaunchKernelGGL(k_take_field<float4>, g, dim3(256), 0, s, src, stride, dst, width, rows, out);
+  else
+    hipLaunchKernelGGL(k_take_field<float>, g, dim3(256), 0, s, src, stride, dst, width, rows, out);
   return hipGetLastError();
 }
 

@@ -135,7 +135,7 @@ struct prc_d2z_ctx {
   int* d_hrange = nullptr;  // lowest and highest occupied history bin
   double* d_pk = nullptr;  // power spectrum bins: counts (uint64) then 3 sums, kPkMaxBins each
   int* d_flag = nullptr;
-  unsigned* d_maxabs = nullptr;  // max |delta| of the input field (float bits)
+  FieldCheck* h_check = nullptr;  // pinned host memory: the blocks' results of the input check
   // history correction: skewer sums and counts per ionized fraction, zcur per
   // fraction, the history in, the corrected history and the per-bin table
   double* d_mfp_sum = nullptr;
@@ -564,6 +564,7 @@ void prc_d2z_destroy(prc_d2z_ctx* c) {
   c->timer.destroy();
   if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
   for (void* q : c->allocs) (void)hipFree(q);
+  if (c->h_check) (void)hipHostFree(c->h_check);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   (void)hipSetDevice(dev);
   delete c;
@@ -682,7 +683,6 @@ int prc_d2z_create(const prc_d2z_params* p, prc_d2z_ctx** out) {
   A_(c->d_hrange, sizeof(int) * 2);
   A_(c->d_pk, sizeof(double) * 4 * kPkMaxBins);
   A_(c->d_flag, sizeof(int));
-  A_(c->d_maxabs, sizeof(unsigned));
   A_(c->d_mfp_sum, sizeof(double) * kNXMfp);
   A_(c->d_mfp_cnt, sizeof(unsigned) * kNXMfp * kNMfp);
   A_(c->d_zcur, sizeof(float) * kNXMfp);
@@ -692,6 +692,9 @@ int prc_d2z_create(const prc_d2z_params* p, prc_d2z_ctx** out) {
   A_(c->d_grfA, sizeof(double));
 #undef A_
   if (e != hipSuccess) return bail(PRC_D2Z_ERR_OOM, std::string("device allocation failed: ") + hipGetErrorString(e));
+  if ((e = hipHostMalloc(reinterpret_cast<void**>(&c->h_check), sizeof(FieldCheck) * kFieldChecks, hipHostMallocDefault)) !=
+      hipSuccess)
+    return bail(PRC_D2Z_ERR_OOM, std::string("pinned host memory: ") + hipGetErrorString(e));
   // twiddle tables and the FP64 scalar set-up, all on the device
   SetupParams sp{p->Omegam, p->Omegab, p->Omegal, p->h,    p->ns,   p->sigma8, p->w, p->BoxSize,
                  p->zInit,  p->Rmin,   p->Rmax,   p->zeta, p->M_min, p->N,      p->Nscales};
@@ -729,18 +732,12 @@ int prc_d2z_create(const prc_d2z_params* p, prc_d2z_ctx** out) {
   return PRC_D2Z_OK;
 }
 
-// The split z pass's input scale from the new field: a power of two <= 256
-// DInit / max|delta| (its stage-A operands stay below 2^16 in FP16; see
-// mfma_split_kernels.hip), at most 2^8.  A changed scale drops the captured
+// The split z pass's input scale from the new field's largest |delta|: a power
+// of two <= 256 DInit / max|delta| (its stage-A operands stay below 2^16 in FP16;
+// see mfma_split_kernels.hip), at most 2^8.  A changed scale drops the captured
 // graph, whose launch arguments hold the old one.
-static int update_zscale(prc_d2z_ctx* c) {
-  if (!use_split(c->p)) return PRC_D2Z_OK;
-  unsigned bits = 0;
-  PRC_CHECK(c, launch_maxabs(c->d_delta, c->ncell, c->d_maxabs, c->stream), "input range");
-  PRC_CHECK(c, hipMemcpyAsync(&bits, c->d_maxabs, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream), "input range");
-  PRC_CHECK(c, hipStreamSynchronize(c->stream), "input range");
-  float mx = 0.0f;
-  memcpy(&mx, &bits, sizeof(mx));
+static void update_zscale(prc_d2z_ctx* c, float mx) {
+  if (!use_split(c->p)) return;
   int e = 8;
   if (mx > 0.0f) e = std::min(8, std::max(-100, (int)std::floor(std::log2(256.0 * (double)c->sc.DInit / mx))));
   const float zs = ldexpf(1.0f, e);
@@ -749,31 +746,64 @@ static int update_zscale(prc_d2z_ctx* c) {
     c->graph_exec = nullptr;
   }
   c->zscale = zs;
+}
+
+// Checks the field in d_delta (src = nullptr), or copies it there from device
+// memory and checks it in the same pass; waits for the stream.
+static int check_field(prc_d2z_ctx* c, const float* src, long long stride, float* mx, bool* finite) {
+  const long long rows = (long long)c->N * c->N;
+  PRC_CHECK(c,
+            launch_take_field(src ? src : c->d_delta, src ? stride : c->N, src ? c->d_delta : nullptr, c->N, rows,
+                              c->h_check, c->stream),
+            "input check");
+  PRC_CHECK(c, hipStreamSynchronize(c->stream), "copy in");
+  unsigned bits = 0;
+  for (int k = 0; k < take_field_blocks(rows * c->N); ++k) bits = std::max(bits, c->h_check[k].maxbits);
+  *finite = bits < 0x7f800000u;
+  memcpy(mx, &bits, sizeof(bits));
   return PRC_D2Z_OK;
+}
+
+// Whether the context's kernels may read `bytes` from src: device memory of its
+// device, all inside one allocation.  Anything else goes through the runtime's
+// copy, which takes it or refuses it.
+static bool readable_here(const prc_d2z_ctx* c, const float* src, size_t bytes) {
+  hipPointerAttribute_t a;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (reinterpret_cast<uintptr_t>(src) % sizeof(float) == 0 && hipPointerGetAttributes(&a, src) == hipSuccess &&
+      a.type == hipMemoryTypeDevice && a.device == c->p.device &&
+      hipMemGetAddressRange(&base, &size, const_cast<float*>(src)) == hipSuccess) {
+    const size_t off = reinterpret_cast<uintptr_t>(src) - reinterpret_cast<uintptr_t>(base);
+    if (off <= size && bytes <= size - off) return true;
+  }
+  (void)hipGetLastError();
+  return false;
 }
 
 static int set_delta_impl(prc_d2z_ctx* c, const float* src, int layout, hipMemcpyKind kind) {
   if (!c || !src) return c ? c->fail(PRC_D2Z_ERR_BAD_ARG, "null field") : PRC_D2Z_ERR_BAD_ARG;
   (void)hipSetDevice(c->p.device);
   const int N = c->N;
-  if (layout == PRC_D2Z_DENSE) {
+  if (layout != PRC_D2Z_DENSE && layout != PRC_D2Z_PADDED) return c->fail(PRC_D2Z_ERR_BAD_ARG, "unknown layout");
+  const long long stride = layout == PRC_D2Z_DENSE ? N : N + 2;
+  // the last row of a padded field ends with its cells
+  const size_t bytes = sizeof(float) * ((size_t)stride * ((size_t)N * N - 1) + N);
+  const bool here = kind == hipMemcpyDeviceToDevice && readable_here(c, src, bytes);
+  if (!here && layout == PRC_D2Z_DENSE)
     PRC_CHECK(c, hipMemcpyAsync(c->d_delta, src, sizeof(float) * c->ncell, kind, c->stream), "copy in");
-  } else if (layout == PRC_D2Z_PADDED) {
+  else if (!here)
     PRC_CHECK(c, hipMemcpy2DAsync(c->d_delta, sizeof(float) * N, src, sizeof(float) * (N + 2), sizeof(float) * N,
                                   (size_t)N * N, kind, c->stream),
               "copy in");
-  } else {
-    return c->fail(PRC_D2Z_ERR_BAD_ARG, "unknown layout");
-  }
-  int bad = 0;
-  PRC_CHECK(c, launch_count_nonfinite(c->d_delta, c->ncell, c->d_flag, c->stream), "input check");
-  PRC_CHECK(c, hipMemcpyAsync(&bad, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream), "input check");
-  PRC_CHECK(c, hipStreamSynchronize(c->stream), "copy in");
+  float mx = 0.0f;
+  bool finite = true;
+  if (int rc = check_field(c, here ? src : nullptr, stride, &mx, &finite)) return rc;
   c->have_delta = false;
   c->have_spectrum = false;
   c->have_result = false;
-  if (bad) return c->fail(PRC_D2Z_ERR_NAN_INPUT, "density field holds NaN or Inf");
-  if (int rc = update_zscale(c)) return rc;
+  if (!finite) return c->fail(PRC_D2Z_ERR_NAN_INPUT, "density field holds NaN or Inf");
+  update_zscale(c, mx);
   c->have_delta = true;
   return PRC_D2Z_OK;
 }
@@ -819,7 +849,12 @@ int prc_d2z_generate_delta(prc_d2z_ctx* c, uint64_t seed, int white_noise_only) 
   PRC_CHECK(c, hipStreamSynchronize(s), "field generation");
   c->timing = was_timing;
   c->have_spectrum = false;
-  if (int rc = update_zscale(c)) return rc;
+  if (use_split(c->p)) {
+    float mx = 0.0f;
+    bool finite = true;
+    if (int rc = check_field(c, nullptr, 0, &mx, &finite)) return rc;
+    update_zscale(c, mx);
+  }
   c->have_delta = true;
   return PRC_D2Z_OK;
 }
