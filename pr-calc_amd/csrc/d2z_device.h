@@ -139,6 +139,17 @@ __device__ __forceinline__ float filter_coef(int m, float dkR, float invN3) {
   return tophat(__builtin_amdgcn_sqrtf((float)m) * dkR) * invN3;
 }
 
+// The table's value for M > 0, without branches
+__device__ __forceinline__ float interpolated_filter(float km, float dkRh, float invN3, const float4* tab, int M) {
+  const float u = km * dkRh;
+  int i = (int)u;
+  i = i < M - 1 ? i : M - 1;
+  const float t = u - (float)i;
+  const float4 c = tab[i];
+  const float w = fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x) * invN3;
+  return km == 0.0f ? 0.0f : w;
+}
+
 // W(|k| R) / N^3 from the interpolation table (entries c0..c3 per interval of
 // length 1/invh in x = |k| R) for |k| = km dk; dkRh = dk R invh.  M = 0 or
 // km = 0 fall back to the exact value / the zeroed mean mode.
@@ -146,12 +157,7 @@ __device__ __forceinline__ float filter_from_table(float km, float dkR, float dk
                                                    const float4* tab, int M) {
   if (km == 0.0f) return 0.0f;
   if (M == 0) return tophat(km * dkR) * invN3;
-  const float u = km * dkRh;
-  int i = (int)u;
-  i = i < M - 1 ? i : M - 1;
-  const float t = u - (float)i;
-  const float4 c = tab[i];
-  return fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x) * invN3;
+  return interpolated_filter(km, dkRh, invN3, tab, M);
 }
 
 // One radius's W table from a |k| table: wt[q] = filter_from_table(kt[q], ...)
@@ -167,14 +173,7 @@ __device__ __forceinline__ void fill_wtable(float* wt, const float* kt, int n, f
     for (int k = 0; k < ITERS; ++k) {
       const int q = tid + k * NT;
       if (q < n) {
-        const float km = kt[q];
-        const float u = km * dkRh;
-        int i = (int)u;
-        i = i < M - 1 ? i : M - 1;
-        const float t = u - (float)i;
-        const float4 c = tab[i];
-        const float w = fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x) * scale;
-        wt[q] = km == 0.0f ? 0.0f : w;
+        wt[q] = interpolated_filter(kt[q], dkRh, scale, tab, M);
       }
     }
   } else {

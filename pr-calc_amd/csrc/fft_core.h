@@ -390,9 +390,15 @@ __device__ __forceinline__ void lds_gather(float2 (&v)[P::E], int i, V lds) {
 // returns.  TAIL = false leaves out the barrier after the last gather: the
 // caller then synchronises before anything rewrites the region (a loop over
 // tiles or radii syncs at the top of its body, which every wave reaches only
-// after its last stage has used the gathered values).
-template <class P, int DIR, int STAGE = 0, class V, bool TWT = false, bool TAIL = true>
-__device__ __forceinline__ void pencil_fft(float2 (&v)[P::E], int i, const float2* __restrict__ tw, V lds) {
+// after its last stage has used the gathered values).  hook() runs after the
+// barrier that follows the first stage (plans of two or more stages), when no
+// wave reads any more what it formed v from.
+struct NoHook {
+  __device__ __forceinline__ void operator()() const {}
+};
+template <class P, int DIR, int STAGE = 0, class V, bool TWT = false, bool TAIL = true, class H = NoHook>
+__device__ __forceinline__ void pencil_fft(float2 (&v)[P::E], int i, const float2* __restrict__ tw, V lds,
+                                           H hook = H{}) {
   if constexpr (STAGE == P::S - 1) {
     stockham_stage<P, STAGE, DIR, true, V, TWT>(v, i, tw, lds);
   } else {
@@ -400,6 +406,7 @@ __device__ __forceinline__ void pencil_fft(float2 (&v)[P::E], int i, const float
     stockham_stage<P, STAGE, DIR, false, V, TWT>(v, i, tw, lds);
     if constexpr (V::kWaveLocal) wave_lds_sync(); else __syncthreads();
     lds_gather<P>(v, i, lds);
+    if constexpr (STAGE == 0) hook();
     if constexpr (TAIL || STAGE + 2 < P::S) {
       if constexpr (!V::kWaveLocal) lds_hold(v);  // the gather is done before the barrier
       if constexpr (V::kWaveLocal) wave_lds_sync(); else __syncthreads();

@@ -438,20 +438,22 @@ __global__ void __launch_bounds__(256)
 // intermediate T_r = Tbuf + r_local * N*N*N/2 (T layout).
 //
 // W depends on kx only through |fx| (fx = kx or kx - N), so per radius the
-// block first tabulates W in LDS for its CF columns and the N/2 + 1 values of
+// block tabulates W in LDS for its CF columns and the N/2 + 1 values of
 // |fx| (half the filter evaluations of a per-element loop), plus the kz = N/2
-// column for the packed slot.  |k| of every table entry is tabulated once
-// before the radius loop.  The table is laid out [|fx|][column] so that the
-// lanes of a wave (consecutive columns, then consecutive kx) read consecutive
-// words.
-// LDS of one fused x block: the padded exchange buffer (float2) and the |k|
-// table (float)
+// column for the packed slot.  A thread keeps |k| of its entries in registers.
+// The table is laid out [|fx|][column] so that the lanes of a wave (consecutive
+// columns, then consecutive kx) read consecutive words.  It has LDS of its own:
+// the next radius's table is filled after the first exchange of this one's
+// transform, while other waves transform, instead of between two barriers of its
+// own with every wave waiting on the same chain of LDS reads.
+// LDS of one fused x block: the padded exchange buffer (float2), the W table
+// (float) and the plan's twiddles (float2)
 template <class P, int CF>
 struct FxLds {
   static constexpr int SH = ilog2(P::radices[0]);
   static constexpr int NROW = P::L + (P::L >> SH);  // padded exchange rows
   static constexpr int SMEM = NROW * CF;           // float2
-  static constexpr int KTAB = (CF + 1) * (P::L / 2 + 1);  // float
+  static constexpr int WTAB = (CF + 1) * (P::L / 2 + 1);  // float
   // the plan's twiddles in LDS (float2); none at N = 2048, where they do not fit
   // beside the largest W(x) table and are read from memory
   static constexpr bool TW = P::L <= 1024;
@@ -461,7 +463,7 @@ struct FxLds {
 // One tile (ky, kz block, column sub-tile) of the fused x pass for nb radii.
 // wsh (the W(x) table, wM intervals) and, with FxLds::TW, tw (the plan's
 // twiddles, transposed) are in LDS and may still be being written: the barrier
-// before the radius loop covers them.  The radius loop reads no global memory
+// before the first fill covers them.  The radius loop reads no global memory
 // but the packed lanes' DN: loads return in order behind the stores that a wave
 // issued before them, so twiddles read from memory made every radius wait for
 // the previous radius's stores (1024^3: 26.8 -> 24.2 ms per 16 radii; N <= 512
@@ -471,20 +473,16 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
                                         const float2* __restrict__ DN, TS* __restrict__ Tbuf, float dk, float invN3,
                                         const RadiusConst* __restrict__ rc, int r0, int nb,
                                         const float2* tw, const float4* wsh, int wM, float winvh, long long tile,
-                                        float2* smem, float* ktab) {
+                                        float2* smem, float* wtab) {
   constexpr int N = P::L, T = P::T, E = P::E;
   constexpr int NSUB = C / CF;
   constexpr int NF = N / 2 + 1;           // distinct |fx|
   constexpr int NT = P::T * CF;           // threads
+  constexpr int NW = (FxLds<P, CF>::WTAB + NT - 1) / NT;  // table entries per thread
   constexpr long long Nh = N / 2;
   constexpr long long plane = (long long)N * N * Nh;
   constexpr int SH = FxLds<P, CF>::SH;
-  constexpr int NROW = FxLds<P, CF>::NROW;
-  // W table [|fx|][CF] then the kz = N/2 column [|fx|]; it aliases the
-  // transform's exchange buffer, which is idle between radii
-  static_assert((CF + 1) * NF <= 2 * NROW * CF, "W table must fit in the exchange buffer");
-  float* wtab = reinterpret_cast<float*>(smem);
-  float* wpk = wtab + CF * NF;
+  float* wpk = wtab + CF * NF;  // W table [|fx|][CF], then the kz = N/2 column [|fx|]
   const int tid = threadIdx.x;
   const int cl = tid % CF, i = tid / CF;
   const int sub = (int)(tile % NSUB);
@@ -507,27 +505,34 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
   TS* tp = Tbuf + (long long)kzb * N * N * C + (long long)kyt * C + sub * CF + cl;  // element x at tp[x*N*C]
   const LdsColPad<SH> lds{smem + cl, CF};
   const int ntab = (has_packed ? CF + 1 : CF) * NF;
-  for (int q = tid; q < ntab; q += NT) {
-    int f, kzq;
-    if (q < CF * NF) {
-      f = q / CF;
-      kzq = kz0 + q % CF;
-    } else {
-      f = q - CF * NF;
-      kzq = N / 2;
-    }
-    ktab[q] = kmag_grid(f * f + fy2 + kzq * kzq);
-  }
-  __syncthreads();  // ktab and the W(x) table complete
-#pragma unroll 1
-  for (int rl = 0; rl < nb; ++rl) {
-    __syncthreads();  // the last radius's final gather is done (pencil_fft without its tail barrier)
+  auto kmag = [&](int q) {  // |k|/dk of table entry q
+    const int f = q < CF * NF ? q / CF : q - CF * NF, kzq = q < CF * NF ? kz0 + q % CF : N / 2;
+    return kmag_grid(f * f + fy2 + kzq * kzq);
+  };
+  float km[NW];
+#pragma unroll
+  for (int k = 0; k < NW; ++k) km[k] = kmag(tid + k * NT);
+  // W(|k| R)/N^3 of radius rl; with an interpolation table (wM > 0) a thread's
+  // entries are independent and written without branches, so their LDS reads
+  // overlap instead of queueing one after the other
+  auto fill = [&](int rl) {
     const float dkR = dk * rc[r0 + rl].R;
     const float dkRh = dkR * winvh;
-    // tabulate W(|k| R)/N^3 for this block's columns (the exchange buffer is
-    // free after the barrier above)
-    fill_wtable<NT, ((CF + 1) * NF + NT - 1) / NT>(wtab, ktab, ntab, dkR, dkRh, invN3, wsh, wM, tid);
-    __syncthreads();
+    if (wM > 0) {
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+        const float w = interpolated_filter(km[k], dkRh, invN3, wsh, wM);
+        if (tid + k * NT < ntab) wtab[tid + k * NT] = w;
+      }
+    } else {
+      for (int q = tid; q < ntab; q += NT) wtab[q] = filter_of_kmag(kmag(q), dkR, invN3);
+    }
+  };
+  __syncthreads();  // the W(x) table and the twiddles are complete
+  fill(0);
+#pragma unroll 1
+  for (int rl = 0; rl < nb; ++rl) {
+    __syncthreads();  // W table complete; the last radius's final gather is done (pencil_fft without its tail barrier)
     float2 v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -542,9 +547,15 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
         v[e] = make_float2(w0 * m[e].x - wn * b.y, w0 * m[e].y + wn * b.x);
       }
     }
-    lds_hold(v);      // the table reads stay above the barrier
-    __syncthreads();  // table reads done before the transform reuses the buffer
-    pencil_fft<P, +1, 0, LdsColPad<SH>, FxLds<P, CF>::TW, false>(v, i, tw, lds);
+    auto next = [&] {
+      if (rl + 1 < nb) fill(rl + 1);
+    };
+    if constexpr (P::S == 1) {  // no exchange: the table reads end here
+      lds_hold(v);
+      __syncthreads();
+      next();
+    }
+    pencil_fft<P, +1, 0, LdsColPad<SH>, FxLds<P, CF>::TW, false>(v, i, tw, lds, next);
     TS* dst = tp + (long long)rl * plane;
 #pragma unroll
     for (int e = 0; e < E; ++e) st(dst, (long long)(i + e * T) * N * C, v[e]);
@@ -557,7 +568,7 @@ __global__ void __launch_bounds__(P::T* CF)
          TS* __restrict__ Tbuf, float dk, float invN3, const RadiusConst* __restrict__ rc, int r0, int nb,
          const float2* __restrict__ tw, const float4* __restrict__ wcoef, int wM, float winvh) {
   __shared__ float2 smem[FxLds<P, CF>::SMEM];
-  __shared__ float ktab[FxLds<P, CF>::KTAB];  // |k|/dk of the table entries, same order
+  __shared__ float wtab[FxLds<P, CF>::WTAB];
   extern __shared__ float4 wsh[];              // W(x) interpolation table (wM intervals)
   __shared__ float2 s_tw[FxLds<P, CF>::NTW];
   for (int q = threadIdx.x; q < wM; q += P::T * CF) wsh[q] = wcoef[q];
@@ -567,7 +578,7 @@ __global__ void __launch_bounds__(P::T* CF)
                              ? line_tile(blockIdx.x, gridDim.x, line_group(C / CF, C * (int)sizeof(TS)))
                              : xcd_tile(blockIdx.x, gridDim.x);
   fx_body<P, C, CF, TS>(S, D0, DN, Tbuf, dk, invN3, rc, r0, nb, FxLds<P, CF>::TW ? s_tw : tw, wsh, wM, winvh, tile,
-                        smem, ktab);
+                        smem, wtab);
 }
 
 // columns per fused-x block: keep the block at <= 512 threads
@@ -901,7 +912,7 @@ constexpr size_t mb_lds_n(MBPass pass) {
     case MBPass::kInvY: return sizeof(float2) * TilePlan<N>::L * Blk<N>::C;
     case MBPass::kFx:
       return sizeof(float2) * (FxLds<PF, FxCols<N>::CF>::SMEM + FxLds<PF, FxCols<N>::CF>::NTW) +
-             sizeof(float) * FxLds<PF, FxCols<N>::CF>::KTAB;
+             sizeof(float) * FxLds<PF, FxCols<N>::CF>::WTAB;
     case MBPass::kFz:
       return sizeof(float2) * (FzLds<PZ>::SMEM + FzLds<PZ>::NTW + PZ::L);
     default: return 0;
@@ -1009,7 +1020,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
   float4* wsh = mb_lds4;
   float2* smem = reinterpret_cast<float2*>(mb_lds4 + maxM);
   float2* s_tw = smem + FxLds<P, CF>::SMEM;
-  float* ktab = reinterpret_cast<float*>(s_tw + FxLds<P, CF>::NTW);
+  float* wtab = reinterpret_cast<float*>(s_tw + FxLds<P, CF>::NTW);
   static_assert(FxLds<P, CF>::TW, "the multi-box x pass keeps its twiddles in LDS");
   int loaded = -1;
   for (long long k = 0;; ++k) {
@@ -1025,7 +1036,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
     }
     float2* T = B.T + (long long)toff * ((long long)N * N * (N / 2));
     fx_body<P, C, CF, float2>(B.S, B.D0, B.DN, T, B.dk, B.invN3, B.rc, r0, nb, s_tw, wsh, B.wM, B.winvh,
-                              t - first[b], smem, ktab);
+                              t - first[b], smem, wtab);
     __syncthreads();
   }
 }
