@@ -565,7 +565,7 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
 template <class P, int C, int CF, class TS>
 __global__ void __launch_bounds__(P::T* CF)
     k_fx(const float2* __restrict__ S, const float2* __restrict__ D0, const float2* __restrict__ DN,
-         TS* __restrict__ Tbuf, float dk, float invN3, const RadiusConst* __restrict__ rc, int r0, int nb,
+         TS* __restrict__ Tbuf, float dk, float invN3, const RadiusConst* __restrict__ rc, int r0, int nb, int nbs,
          const float2* __restrict__ tw, const float4* __restrict__ wcoef, int wM, float winvh) {
   __shared__ float2 smem[FxLds<P, CF>::SMEM];
   __shared__ float wtab[FxLds<P, CF>::WTAB];
@@ -577,8 +577,10 @@ __global__ void __launch_bounds__(P::T* CF)
   const long long tile = std::is_same<TS, float2>::value
                              ? line_tile(blockIdx.x, gridDim.x, line_group(C / CF, C * (int)sizeof(TS)))
                              : xcd_tile(blockIdx.x, gridDim.x);
-  fx_body<P, C, CF, TS>(S, D0, DN, Tbuf, dk, invN3, rc, r0, nb, FxLds<P, CF>::TW ? s_tw : tw, wsh, wM, winvh, tile,
-                        smem, wtab);
+  // gridDim.y > 1 (small grids): block row y takes the nbs radii from y nbs on
+  const int q0 = (int)blockIdx.y * nbs;
+  fx_body<P, C, CF, TS>(S, D0, DN, Tbuf + q0 * ((long long)P::L * P::L * (P::L / 2)), dk, invN3, rc, r0 + q0,
+                        min(nbs, nb - q0), FxLds<P, CF>::TW ? s_tw : tw, wsh, wM, winvh, tile, smem, wtab);
 }
 
 // columns per fused-x block: keep the block at <= 512 threads
@@ -1399,6 +1401,7 @@ static hipError_t filter_impl(const float2* S, const float2* D0, const float2* D
   return hipGetLastError();
 }
 
+constexpr long long kFxBlocks = 2048;
 template <int N, class TS>
 static hipError_t fx_impl(const float2* S, const float2* D0, const float2* DN, TS* Tbuf, float dk, float invN3,
                           const RadiusConst* rc, int r0, int nb, const float2* tw, const WTable& wt,
@@ -1406,8 +1409,14 @@ static hipError_t fx_impl(const float2* S, const float2* D0, const float2* DN, T
   using P = typename FxPlan<N>::P;
   constexpr int C = FxCols<N>::C, CF = FxCols<N>::CF;
   const long long nblk = (long long)N * ((N / 2) / C) * (C / CF);
-  hipLaunchKernelGGL((k_fx<P, C, CF, TS>), dim3((unsigned)nblk), dim3(P::T * CF), sizeof(float4) * wt.M, s, S, D0,
-                     DN, Tbuf, dk, invN3, rc, r0, nb, tw, wt.coef, wt.M, wt.invh);
+  // A small grid has few tiles (128 blocks at N = 64, 512 at 128, for 256 CUs): up
+  // to 2048 blocks share the radii.  x pass at 64^3 x 8: 21 -> 13 us, 128^3 x 32:
+  // 107 -> 91 us (97 with up to 4096 blocks, whose set-up costs more, 115 with
+  // 8192); 192^3 and 256^3 gain nothing from 2 and lose from 4.
+  const int split = (int)std::min<long long>(nb, std::max<long long>(1, kFxBlocks / nblk));
+  const int nbs = (nb + split - 1) / split;
+  hipLaunchKernelGGL((k_fx<P, C, CF, TS>), dim3((unsigned)nblk, (nb + nbs - 1) / nbs), dim3(P::T * CF),
+                     sizeof(float4) * wt.M, s, S, D0, DN, Tbuf, dk, invN3, rc, r0, nb, nbs, tw, wt.coef, wt.M, wt.invh);
   return hipGetLastError();
 }
 
