@@ -263,13 +263,39 @@ __device__ __forceinline__ double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
-// The same in float: the FP16-storage paths sum their per-radius squares over
-// a wave in float (64 lanes; relative error far below their own) and widen to
-// double for the sums over waves and blocks
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// Sums over the 16 lanes of each row of a wave, in every lane, by DPP moves
+// (lanes l ^ 1, l ^ 2, 7 - l and 15 - l of the row): no LDS traffic, where a sum
+// over the wave by shuffles is a chain of six LDS round trips.
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, false),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, false));
+}
+template <class F>
+__device__ __forceinline__ F row_sum(F v) {
+  v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_mov<0x141>(v);  // row_half_mirror
+  v += dpp_mov<0x140>(v);  // row_mirror
   return v;
+}
+// the sum over a wave in float (the matrix-core z passes' squares; relative error
+// far below their own)
+__device__ __forceinline__ float wave_sum_f(float v) {
+  v = row_sum(v);
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+// Adds this lane's acc to the radius's sums in LDS, one slot per row of a wave:
+// FP32 storage sums the rows in double (as GetMeanSigma), FP16 storage in float
+// (relative error far below its own)
+__device__ __forceinline__ void add_squares(double* slots, float acc, bool half, int lane) {
+  const double s = half ? (double)row_sum(acc) : row_sum((double)acc);
+  if ((lane & 15) == 0) atomicAdd(&slots[lane >> 4], s);
 }
 
 // ------------------------------------------------------ FP16 complex pairs

@@ -19,6 +19,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "d2z_device.h"
@@ -624,10 +625,11 @@ struct FxCols {
 // maximum over the batch stays in registers (first radius wins ties) and
 // zreion (and rbubble) is read and written once per batch.  Per-radius sums of
 // delta_R^2 (float products, double sums as GetMeanSigma; with FP16 storage
-// the wave's own sum is float) are kept per wave in
-// LDS and written as one partial per block and radius.
+// the sums of 16 lanes are float) are kept per row of 16 lanes in LDS and
+// written as one partial per block and radius.
 // LDS of one fused z block: the pencil rows, the per-wave sums, the plan's
 // twiddles (transposed) and the c2r glue constants
+constexpr int kFzRed = 16;  // sums per radius: 4 waves x 4 rows of lanes
 template <class P>
 struct FzLds {
   static constexpr int NTW = plan_tw_size<P>() > 0 ? plan_tw_size<P>() : 1;
@@ -638,12 +640,12 @@ struct FzLds {
 // (FP32 storage) or the packed FP16 glue constants (FP16 storage).  A barrier
 // must follow before fz_group reads them.
 template <class P, class TS>
-__device__ __forceinline__ void fz_tables(double (*red)[kFusedMaxRadii], float2* s_twh, float2* s_twf,
+__device__ __forceinline__ void fz_tables(double (*red)[kFzRed], float2* s_twh, float2* s_twf,
                                           const float2* __restrict__ tw_half, const float2* __restrict__ tw_full) {
   constexpr int L = P::L;
   constexpr bool kH = std::is_same<TS, __half2>::value;
   const int t = threadIdx.x;
-  if (t < 4 * kFusedMaxRadii) red[t / kFusedMaxRadii][t % kFusedMaxRadii] = 0.0;
+  for (int q = t; q < kFusedMaxRadii * kFzRed; q += 256) red[q / kFzRed][q % kFzRed] = 0.0;
   copy_twiddles_transposed<P>(s_twh, tw_half, t, 256);
   uint2* const s_pq = reinterpret_cast<uint2*>(s_twf);
   for (int q = t; q < L; q += 256) {
@@ -658,20 +660,23 @@ __device__ __forceinline__ void fz_tables(double (*red)[kFusedMaxRadii], float2*
 // row's intermediates are transformed in turn, d2z() is evaluated per cell,
 // the maximum over the batch stays in registers (first radius wins ties) and
 // zreion (and rbubble) is read and written once.  Per-radius sums of
-// delta_R^2 (float products, double sums as GetMeanSigma; with FP16 storage
-// the wave's own sum is float) are added per wave into red.  F32B: the
-// barrier as one FP32 FMA (barrier_z_f32), as for FP16 storage, instead of the
+// delta_R^2 (add_squares) go into red, unscaled.  F32B: the barrier as one FP32 FMA (barrier_z_f32), as for FP16 storage, instead of the
 // reference's double evaluation (the mixed path's FP32 intermediates).
-template <class P, int C, bool RB, class TS, bool F32B = false>
+//
+// G > 1: the block's G groups of 256 threads take the same rows and each its own
+// contiguous part of the radii (iters of them at most; nb may be less, also 0,
+// for the last groups, whose remaining rounds count for nothing), and group 0
+// joins the maxima through join (LDS, (G - 1) x 256 x E pairs).
+template <class P, int C, bool RB, class TS, bool F32B = false, int G = 1>
 __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __restrict__ zre,
                                          float* __restrict__ rbub, long long nrows,
                                          const RadiusConst* __restrict__ rc, int r0, int nb, float iscale,
                                          long long base, const float2* s_twh, const float2* s_twf, float2* smem,
-                                         double (*red)[kFusedMaxRadii]) {
+                                         double (*red)[kFzRed], int iters = 0, float2* join = nullptr) {
   constexpr int L = P::L, T = P::T, E = P::E;
   constexpr bool kH = std::is_same<TS, __half2>::value;
   const uint2* const s_pq = reinterpret_cast<const uint2*>(s_twf);
-  const int t = threadIdx.x;
+  const int t = threadIdx.x % 256;
   const int i = t % T, rr = t / T;
   const int w = t >> 6, lane = t & 63;
   const long long plane = nrows * L;
@@ -682,7 +687,7 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
   // for FP16 at N = 2048.
   using Lds = LdsRow<L, kH && (E <= 8)>;
   const Lds lds{smem + rr * Lds::STRIDE};
-  const double sc = (double)iscale, sc2 = sc * sc;
+  const double sc = (double)iscale;
   const long long row = base + rr;
   const bool valid = row < nrows;
   const long long r = TLay<2 * L, TS>::row(valid ? row : 0);
@@ -694,24 +699,27 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
     bR0[e] = 0.f;
     bR1[e] = 0.f;
   }
-  // FP32 storage at N = 1024 (8-element pencils), no bubble radii: the next
-  // radius's row is loaded while this one is transformed (16 more VGPRs, 112
-  // -> 124, still 4 waves per SIMD; z pass 110 -> 107.5 ms per 1024^3 x 96
-  // step, same bits).  The other variants would lose a wave per SIMD.
-  constexpr bool kPre = !kH && !RB && E <= 8 && L == 512;
+  // FP32 storage at N = 1024 and 128 (8-element pencils), no bubble radii: the
+  // next radius's row is loaded while this one is transformed (16 more VGPRs,
+  // still 4 waves per SIMD; z pass 110 -> 107.5 ms per 1024^3 x 96 step, same
+  // bits).  The other variants would lose a wave per SIMD.
+  constexpr bool kPre = !kH && !RB && E <= 8 && (L == 512 || L == 64);
   float2 nx[kPre ? E : 1];
   if constexpr (kPre) {
 #pragma unroll
     for (int e = 0; e < E; ++e) nx[e] = ld(Tbuf, zrow_offset<P, C>(i, e, r, nrows));
   }
+  const int last = G > 1 ? max(nb - 1, 0) : nb - 1;  // the extra rounds repeat a radius
 #pragma unroll 1
-  for (int q = 0; q < nb; ++q) {
+  for (int q1 = 0; q1 < (G > 1 ? iters : nb); ++q1) {
+    const int q = G > 1 ? min(q1, last) : q1;
+    const bool live = G == 1 || q1 < nb;
     const TS* tp = Tbuf + (long long)q * plane;
     float2 v[E];
     if constexpr (kPre) {
 #pragma unroll
       for (int e = 0; e < E; ++e) v[e] = nx[e];
-      const TS* tn = Tbuf + (long long)min(q + 1, nb - 1) * plane;  // the last radius reloads its own row
+      const TS* tn = Tbuf + (long long)min(q + 1, last) * plane;  // the last radius reloads its own row
 #pragma unroll
       for (int e = 0; e < E; ++e) nx[e] = ld(tn, zrow_offset<P, C>(i, e, r, nrows));
     }
@@ -742,6 +750,7 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
     // the output scale iscale (a power of two) is applied inside the
     // barrier's FMA and to the sum of squares, where it is exact (the FP16
     // storage and F32B evaluate it in FP32: |error| <= (|z| + |A B - 1|) 2^-24)
+    if (G > 1 && !live) continue;  // the last barrier of a round is in the transform
     const double A = rc[r0 + q].A, B = rc[r0 + q].B;
     const BarrierF32 bk = barrier_f32(A, B, iscale);
     const float R = rc[r0 + q].R;
@@ -766,8 +775,26 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
         best[e].y = zmax_nonneg(best[e].y, z1);
       }
     }
-    const double wsum = kH ? (double)wave_sum_f(valid ? acc : 0.0f) * sc2 : wave_sum(valid ? (double)acc * sc2 : 0.0);
-    if (lane == 0) red[w][q] += wsum;
+    add_squares(red[q] + 4 * w, valid ? acc : 0.0f, kH, lane);
+  }
+  if constexpr (G > 1) {
+    static_assert(!RB, "bubble radii are not joined");
+    const int g = threadIdx.x / 256;
+    if (g > 0) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) join[((g - 1) * E + e) * 256 + t] = best[e];
+    }
+    __syncthreads();
+    if (g == 0) {
+      for (int k = 0; k < G - 1; ++k)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const float2 b = join[(k * E + e) * 256 + t];
+          best[e] = make_float2(zmax_nonneg(best[e].x, b.x), zmax_nonneg(best[e].y, b.y));
+        }
+    }
+    __syncthreads();  // join is written again for the next rows
+    if (g > 0) return;
   }
   if (valid) {
     float2* zp = reinterpret_cast<float2*>(zre + row * (2 * L));
@@ -788,33 +815,46 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
   }
 }
 
+// Groups of 256 threads per fused z block.  The rows of a small grid are few
+// waves (256 at N = 64, 2048 at 128), each on a chain of all the batch's radii
+// with the chip mostly idle; the groups share the chain.  z pass at 64^3 x 8 with
+// 1, 2, 4 groups: 18, 14, 13 us; 128^3 x 32: 61, 56, 64 us in FP32 and 61, 43, 43
+// in FP16.  (Blocks of their own for parts of the radii, joined by integer maxima
+// on zreion in memory, took 52 us at 64^3: the atomics.)
+constexpr int fz_groups(int N, bool rb) { return rb ? 1 : (N <= 64 ? 4 : (N == 128 ? 2 : 1)); }
+
 // The fused z pass (c2r + barrier + running max) over all rows: a
 // grid-stride kernel over row groups; one partial sum per block and radius.
 template <class P, int C, bool RB, class TS, bool F32B = false>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256 * fz_groups(2 * P::L, RB))
     k_fz(const TS* __restrict__ Tbuf, float* __restrict__ zre, float* __restrict__ rbub, long long nrows,
          const RadiusConst* __restrict__ rc, int r0, int nb, double* __restrict__ partial, float iscale,
          const float2* __restrict__ tw_half, const float2* __restrict__ tw_full) {
-  constexpr int ROWS = 256 / P::T;
-  __shared__ float2 smem[FzLds<P>::SMEM];
-  __shared__ double red[4][kFusedMaxRadii];
+  constexpr int ROWS = 256 / P::T, G = fz_groups(2 * P::L, RB);
+  __shared__ float2 smem[G * FzLds<P>::SMEM];
+  __shared__ float2 join[G > 1 ? (G - 1) * 256 * P::E : 1];
+  __shared__ double red[kFusedMaxRadii][kFzRed];
   // twiddles in LDS (the blocks are persistent: copied once), the plan's
   // stages transposed so that lanes with consecutive k read consecutive words;
   // c2r glue: w^k for FP32 storage, the packed FP16 constants (P, Q) of
   // c2r_glue_h2 for FP16 storage
   __shared__ float2 s_twh[FzLds<P>::NTW];
   __shared__ float2 s_twf[P::L];
-  fz_tables<P, TS>(red, s_twh, s_twf, tw_half, tw_full);
+  const int g = threadIdx.x / 256, iters = (nb + G - 1) / G;
+  const int q0 = min(g * iters, nb - 1), n = max(0, min(iters, nb - g * iters));  // this group's radii
+  const TS* T0 = Tbuf + (long long)q0 * nrows * P::L;
+  if (g == 0) fz_tables<P, TS>(red, s_twh, s_twf, tw_half, tw_full);
   __syncthreads();
 #pragma unroll 1
   for (long long base = (long long)blockIdx.x * ROWS; base < nrows; base += (long long)gridDim.x * ROWS)
-    fz_group<P, C, RB, TS, F32B>(Tbuf, zre, rbub, nrows, rc, r0, nb, iscale, base, s_twh, s_twf, smem, red);
+    fz_group<P, C, RB, TS, F32B, G>(T0, zre, rbub, nrows, rc, r0 + q0, n, iscale, base, s_twh, s_twf,
+                                    smem + g * FzLds<P>::SMEM, red + q0, iters, join);
   __syncthreads();
   const int t = threadIdx.x;
   if (t < nb) {
     double s = 0.0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); ++k) s += red[k][t];
-    partial[(long long)(r0 + t) * gridDim.x + blockIdx.x] = s;
+    for (int k = 0; k < kFzRed; ++k) s += red[t][k];
+    partial[(long long)(r0 + t) * gridDim.x + blockIdx.x] = s * ((double)iscale * (double)iscale);
   }
 }
 
@@ -1054,7 +1094,7 @@ __global__ void __launch_bounds__(256) k_mb_fz(const MBox* __restrict__ boxes, c
   __shared__ float2 smem[FzLds<P>::SMEM];
   __shared__ float2 s_twh[FzLds<P>::NTW];
   __shared__ float2 s_twf[P::L];
-  __shared__ double red[4][kFusedMaxRadii];
+  __shared__ double red[kFusedMaxRadii][kFzRed];
   const long long G = gridDim.x;
   for (int q = threadIdx.x; q < nbox * nb; q += 256)
     boxes[q / nb].part[(long long)(r0 + q % nb) * G + blockIdx.x] = 0.0;
@@ -1062,7 +1102,7 @@ __global__ void __launch_bounds__(256) k_mb_fz(const MBox* __restrict__ boxes, c
     __syncthreads();
     if ((int)threadIdx.x < nb) {
       double s = 0.0;
-      for (int w = 0; w < 4; ++w) s += red[w][threadIdx.x];
+      for (int w = 0; w < kFzRed; ++w) s += red[threadIdx.x][w];
       boxes[b].part[(long long)(r0 + threadIdx.x) * G + blockIdx.x] = s;
     }
     __syncthreads();
@@ -1431,16 +1471,16 @@ static int fz_grid(bool half, bool rb, bool fbar) {
   int dev = 0, cus = 0, per_cu = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  auto occ = [&](auto kern) {
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256 * fz_groups(N, rb), 0);
+  };
   if (e == hipSuccess) {
     if (half)
-      e = rb ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, true, __half2>, 256, 0)
-             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, false, __half2>, 256, 0);
+      e = rb ? occ(k_fz<P, C, true, __half2>) : occ(k_fz<P, C, false, __half2>);
     else if (fbar)
-      e = rb ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, true, float2, true>, 256, 0)
-             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, false, float2, true>, 256, 0);
+      e = rb ? occ(k_fz<P, C, true, float2, true>) : occ(k_fz<P, C, false, float2, true>);
     else
-      e = rb ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, true, float2>, 256, 0)
-             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fz<P, C, false, float2>, 256, 0);
+      e = rb ? occ(k_fz<P, C, true, float2>) : occ(k_fz<P, C, false, float2>);
   }
   long long g = (e == hipSuccess && cus > 0 && per_cu > 0) ? (long long)cus * per_cu : 2048;
   if (g > kFzMaxBlocks) g = kFzMaxBlocks;
@@ -1454,24 +1494,14 @@ static hipError_t fz_impl(const TS* Tbuf, float* zre, float* rbub, const RadiusC
   using P = Plan<N / 2>;
   constexpr int C = Blk<N>::C;
   const long long nrows = (long long)N * N;
-  if constexpr (std::is_same<TS, float2>::value) {
-    if (fbar) {
-      if (rbub)
-        hipLaunchKernelGGL((k_fz<P, C, true, TS, true>), dim3(nblk), dim3(256), 0, s, Tbuf, zre, rbub, nrows, rc, r0,
-                           nb, partial, iscale, twh, twf);
-      else
-        hipLaunchKernelGGL((k_fz<P, C, false, TS, true>), dim3(nblk), dim3(256), 0, s, Tbuf, zre, rbub, nrows, rc, r0,
-                           nb, partial, iscale, twh, twf);
-      return hipGetLastError();
-    }
-  }
-  if (rbub)
-    hipLaunchKernelGGL((k_fz<P, C, true, TS>), dim3(nblk), dim3(256), 0, s, Tbuf, zre, rbub, nrows, rc, r0, nb,
-                       partial, iscale, twh, twf);
-  else
-    hipLaunchKernelGGL((k_fz<P, C, false, TS>), dim3(nblk), dim3(256), 0, s, Tbuf, zre, rbub, nrows, rc, r0, nb,
-                       partial, iscale, twh, twf);
-  return hipGetLastError();
+  auto go = [&](auto kern, bool rb) {
+    hipLaunchKernelGGL(kern, dim3(nblk), dim3(256 * fz_groups(N, rb)), 0, s, Tbuf, zre, rbub, nrows, rc, r0, nb, partial,
+                       iscale, twh, twf);
+    return hipGetLastError();
+  };
+  if constexpr (std::is_same<TS, float2>::value)
+    if (fbar) return rbub ? go(k_fz<P, C, true, TS, true>, true) : go(k_fz<P, C, false, TS, true>, false);
+  return rbub ? go(k_fz<P, C, true, TS>, true) : go(k_fz<P, C, false, TS>, false);
 }
 
 int block_width(int N) {
