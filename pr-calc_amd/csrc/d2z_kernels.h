@@ -125,7 +125,8 @@ hipError_t launch_fwd_z(int N, const float* in, float2* out, float dinit, const 
 hipError_t launch_inv_z(int N, const float2* in, float* out, const float2* twh, const float2* twf, hipStream_t s);
 hipError_t launch_tile(int N, int dir, const float2* in, float2* out, const TileMap& mp, const float2* tw,
                        hipStream_t s);
-hipError_t launch_unpack(int N, const float2* S, float2* D0, float2* DN, hipStream_t s);
+// zre, rb (nullptr: none): N^3 floats each that are set to 0 in the same launch
+hipError_t launch_unpack(int N, const float2* S, float2* D0, float2* DN, float* zre, float* rb, hipStream_t s);
 hipError_t launch_filter(int N, const float2* S, const float2* D0, const float2* DN, float2* out, float dkR,
                          float invN3, hipStream_t s);
 // i k_a / |k|^2 * scale * S, component a = axis (0, 1, 2), k = n dk (the

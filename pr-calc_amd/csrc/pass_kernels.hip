@@ -258,9 +258,18 @@ __global__ void __launch_bounds__(256) k_inv_z(const TS* __restrict__ in, float*
 // ------------------------------------------------- unpack after forward
 // D0(k) = (P(k) + conj P(-k))/2,  DN(k) = -i (P(k) - conj P(-k))/2 with P the
 // packed kz = 0 slot of S; D0/DN indexed [kx][ky].
+// A run's start of zreion (and rbubble) from 0 goes along in the same launch (zre,
+// rb: nullptr without); the grid covers N^2 points.
 template <int C>
-__global__ void k_unpack(const float2* __restrict__ S, float2* __restrict__ D0, float2* __restrict__ DN, int N) {
+__global__ void __launch_bounds__(256) k_unpack(const float2* __restrict__ S, float2* __restrict__ D0, float2* __restrict__ DN, int N,
+                                                float4* __restrict__ zre, float4* __restrict__ rb) {
   const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long n4 = (long long)N * N * N / 4, step = (long long)gridDim.x * blockDim.x;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (zre)
+    for (long long q = id; q < n4; q += step) zre[q] = zero;
+  if (rb)
+    for (long long q = id; q < n4; q += step) rb[q] = zero;
   if (id >= (long long)N * N) return;
   const int kx = (int)(id / N), ky = (int)(id % N);
   const int mx = (N - kx) % N, my = (N - ky) % N;
@@ -1404,9 +1413,10 @@ static hipError_t tile_ip_impl(TS* d, const TileMap& mp, float oscale, const flo
 }
 
 template <int N>
-static hipError_t unpack_impl(const float2* S, float2* D0, float2* DN, hipStream_t s) {
+static hipError_t unpack_impl(const float2* S, float2* D0, float2* DN, float* zre, float* rb, hipStream_t s) {
   const long long n = (long long)N * N;
-  hipLaunchKernelGGL((k_unpack<Blk<N>::C>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, S, D0, DN, N);
+  hipLaunchKernelGGL((k_unpack<Blk<N>::C>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, S, D0, DN, N,
+                     reinterpret_cast<float4*>(zre), reinterpret_cast<float4*>(rb));
   return hipGetLastError();
 }
 
@@ -1622,11 +1632,11 @@ hipError_t launch_tile_h(int N, void* data, const TileMap& mp, float oscale, con
   }
 }
 
-hipError_t launch_unpack(int N, const float2* S, float2* D0, float2* DN, hipStream_t s) {
+hipError_t launch_unpack(int N, const float2* S, float2* D0, float2* DN, float* zre, float* rb, hipStream_t s) {
   switch (N) {
 #define X(NN) \
   case NN:    \
-    return unpack_impl<NN>(S, D0, DN, s);
+    return unpack_impl<NN>(S, D0, DN, zre, rb, s);
     PRC_FOR_EACH_N(X)
 #undef X
     default:

@@ -199,7 +199,8 @@ hipError_t timed(prc_d2z_ctx* c, const char* name, F&& f) {
     if (e_ != hipSuccess) return (ctx)->hip_fail(e_, what); \
   } while (0)
 
-int forward(prc_d2z_ctx* c, float dinit) {
+// start: zreion (and rbubble) set to 0 for a run that begins
+int forward(prc_d2z_ctx* c, float dinit, bool start = false) {
   const int N = c->N;
   hipStream_t s = c->stream;
   float2* T0 = c->d_T;
@@ -212,7 +213,11 @@ int forward(prc_d2z_ctx* c, float dinit) {
             "forward y pass");
   PRC_CHECK(c, timed(c, "fwd_x", [&] { return launch_tile(N, -1, T0, c->d_S, xm, c->d_st_full, s); }),
             "forward x pass");
-  PRC_CHECK(c, timed(c, "unpack", [&] { return launch_unpack(N, c->d_S, c->d_D0, c->d_DN, s); }), "unpack");
+  float* rb = start && c->p.RecordBubbleSizes ? c->d_rb : nullptr;
+  PRC_CHECK(c, timed(c, "unpack", [&] {
+              return launch_unpack(N, c->d_S, c->d_D0, c->d_DN, start ? c->d_zre : nullptr, rb, s);
+            }),
+            "unpack");
   c->have_spectrum = true;
   return PRC_D2Z_OK;
 }
@@ -353,10 +358,8 @@ int fused_serial(prc_d2z_ctx* c) {
 // All launches of one run (forward transform through the last radius).
 int enqueue_run(prc_d2z_ctx* c) {
   hipStream_t s = c->stream;
-  int rc = forward(c, c->sc.DInit);
+  int rc = forward(c, c->sc.DInit, true);
   if (rc) return rc;
-  PRC_CHECK(c, launch_fill(c->d_zre, c->ncell, 0.0f, s), "zreion init");
-  if (c->p.RecordBubbleSizes) PRC_CHECK(c, launch_fill(c->d_rb, c->ncell, 0.0f, s), "rbubble init");
   const int NS = c->p.Nscales;
   const double invN3 = 1.0 / ((double)c->N * c->N * c->N);
   if (c->p.mode == PRC_D2Z_PLAIN_FP32) {
