@@ -160,27 +160,6 @@ __device__ __forceinline__ float filter_from_table(float km, float dkR, float dk
   return interpolated_filter(km, dkRh, invN3, tab, M);
 }
 
-// One radius's W table from a |k| table: wt[q] = filter_from_table(kt[q], ...)
-// for q < n, ITERS strided entries per thread of NT (ITERS NT >= n).  With an
-// interpolation table (M > 0) a thread's entries are independent and written
-// without branches, so their LDS reads overlap instead of queueing one after
-// the other; the values are filter_from_table's bit for bit.
-template <int NT, int ITERS>
-__device__ __forceinline__ void fill_wtable(float* wt, const float* kt, int n, float dkR, float dkRh, float scale,
-                                            const float4* tab, int M, int tid) {
-  if (ITERS <= 8 && M > 0) {
-#pragma unroll
-    for (int k = 0; k < ITERS; ++k) {
-      const int q = tid + k * NT;
-      if (q < n) {
-        wt[q] = interpolated_filter(kt[q], dkRh, scale, tab, M);
-      }
-    }
-  } else {
-    for (int q = tid; q < n; q += NT) wt[q] = filter_from_table(kt[q], dkR, dkRh, scale, tab, M);
-  }
-}
-
 // The same in two steps for tables that reuse |k| over radii:
 // kmag_grid(m) = |k| / dk, filter_of_kmag(kmag_grid(m), dkR, invN3) ==
 // filter_coef(m, dkR, invN3) bit for bit.
@@ -188,6 +167,38 @@ __device__ __forceinline__ float kmag_grid(int m) { return __builtin_amdgcn_sqrt
 __device__ __forceinline__ float filter_of_kmag(float km, float dkR, float invN3) {
   if (km == 0.0f) return 0.0f;
   return tophat(km * dkR) * invN3;
+}
+
+// One radius's W table of a matrix x pass block (N points, CF columns from kz0 on,
+// NT threads): wt[f CF + c] = scale W at (|fx| = f, kz0 + c), f <= N/2, and, PK, the
+// kz = N/2 column behind them.  A thread keeps its column, so |k| is two integer
+// operations and a square root on the way to the table read; the values are
+// filter_from_table's bit for bit.
+template <int N, int CF, int NT, bool PK>
+__device__ __forceinline__ void fill_wcolumns(float* wt, int fy2, int kz0, float dkR, float dkRh, float scale,
+                                              const float4* tab, int M, int tid) {
+  constexpr int NF = N / 2 + 1, FS = NT / CF, K = (NF - 1) / FS;
+  static_assert(K * FS == NF - 1, "whole rounds of f, then f = N/2");
+  const int kz = kz0 + tid % CF, f0 = tid / CF, m0 = fy2 + kz * kz, mp = fy2 + (N / 2) * (N / 2);
+  if (M > 0) {
+    float v[K];  // all read before the first is written: the compiler may not reorder these
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int f = f0 + k * FS;
+      v[k] = interpolated_filter(kmag_grid(f * f + m0), dkRh, scale, tab, M);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) wt[tid + k * NT] = v[k];
+    if (tid < CF) wt[tid + K * NT] = interpolated_filter(kmag_grid((NF - 1) * (NF - 1) + m0), dkRh, scale, tab, M);
+    if (PK)
+      for (int f = tid; f < NF; f += NT) wt[CF * NF + f] = interpolated_filter(kmag_grid(f * f + mp), dkRh, scale, tab, M);
+  } else {
+#pragma unroll 1
+    for (int q = tid; q < (PK ? CF + 1 : CF) * NF; q += NT) {
+      const int f = q < CF * NF ? q / CF : q - CF * NF;
+      wt[q] = filter_of_kmag(kmag_grid(f * f + (q < CF * NF ? m0 : mp)), dkR, scale);
+    }
+  }
 }
 
 // ------------------------------------------- per-radius barrier offset B_R

@@ -31,6 +31,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "d2z_device.h"
 #include "d2z_kernels.h"
 #include "fft_core.h"
@@ -160,13 +162,12 @@ __global__ void __launch_bounds__(kFxThreads)
   constexpr long long Nh = kN / 2;
   constexpr long long plane = (long long)kN * kN * Nh;
   __shared__ float2 bufX[kN * kCF];
-  __shared__ float wtab[(kCF + 1) * kNF];  // [|fx|][column], then the kz = N/2 column
-  __shared__ float ktab[(kCF + 1) * kNF];  // |k|/dk of the same entries
+  constexpr int kWT = (kCF + 1) * kNF;
+  __shared__ float wtab[2][kWT];  // of two radii: [|fx|][column], then the kz = N/2 column
   __shared__ float s_max[kFxThreads / 64];
   __shared__ half8_t s_gA[2][2][64];  // the 16-point DFT (stage A), [block h][hi/lo][lane]
   __shared__ float2 s_twc[3 * 256];   // exp(2 pi i m / 1024), m < 768 (stage C)
   extern __shared__ float4 wsh[];     // W(x) interpolation table (wM intervals)
-  float* wpk = wtab + kCF * kNF;
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
@@ -210,18 +211,6 @@ __global__ void __launch_bounds__(kFxThreads)
   for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
   if (l == 0) s_max[w] = mx;
   const int fy2 = fsq(ky, kN);
-  const int ntab = (has_packed ? kCF + 1 : kCF) * kNF;
-  for (int q = tid; q < ntab; q += kFxThreads) {
-    int f, kzq;
-    if (q < kCF * kNF) {
-      f = q / kCF;
-      kzq = kz0 + q % kCF;
-    } else {
-      f = q - kCF * kNF;
-      kzq = kN / 2;
-    }
-    ktab[q] = kmag_grid(f * f + fy2 + kzq * kzq);
-  }
   for (int q = tid; q < wM; q += kFxThreads) wsh[q] = wcoef[q];
   const int qbase = sel ? 2 : 0;
   __syncthreads();
@@ -239,117 +228,133 @@ __global__ void __launch_bounds__(kFxThreads)
   const int kyt = ky ^ TLay<kN, float2>::swap(w);
   float2* tp = Tbuf + (long long)kzb * kN * kN * kC + (long long)kyt * kC + sub * kCF + c;
 
+  // The W table is double-buffered: the next radius's is filled beside stages B
+  // and C, whose stores it overlaps.  Blocks without the packed column (63 of
+  // 64) take a loop without it: a branch per value made each wait for its own
+  // LDS read.  1024^3 x 32: 43.6-44.5 -> 39.1-39.4 ms.
+  auto radii = [&](auto pk) {
+    constexpr bool PK = decltype(pk)::value;
+    auto fill = [&](int rl) {
+      const float dkR = dk * rc[r0 + rl].R;
+      fill_wcolumns<kN, kCF, kFxThreads, PK>(wtab[rl & 1], fy2, kz0, dkR, dkR * winvh, wscale, wsh, wM, tid);
+    };
+    fill(0);
 #pragma unroll 1
-  for (int rl = 0; rl < nb; ++rl) {
-    int zo = 0;  // opaque zero: the LDS operand reads stay inside the radius loop
-    asm volatile("" : "+v"(zo));
-    const float dkR = dk * rc[r0 + rl].R;
-    const float dkRh = dkR * winvh;
-    fill_wtable<kFxThreads, ((kCF + 1) * kNF + kFxThreads - 1) / kFxThreads>(wtab, ktab, ntab, dkR, dkRh, wscale, wsh,
-                                                                              wM, tid);
-    __syncthreads();  // (1) W table complete; the previous radius's stage-B reads of bufX are done
-    // stage A: filter, split, radix 16 on the matrix cores, outputs to bufX
+    for (int rl = 0; rl < nb; ++rl) {
+      int zo = 0;  // opaque zero: the LDS operand reads stay inside the radius loop
+      asm volatile("" : "+v"(zo));
+      const float* wt = wtab[rl & 1];
+      __syncthreads();  // (1) W table complete; the previous radius's stage-B reads of bufX are done
+      // stage A: filter, split, radix 16 on the matrix cores, outputs to bufX
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int b = 4 * w + 2 * t + sel;
-      float2 x[4];
+      for (int t = 0; t < 2; ++t) {
+        const int b = 4 * w + 2 * t + sel;
+        float2 x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int kx = b + 64 * (4 * g + j);
-        const int fa = (kx <= kN / 2) ? kx : kN - kx;
-        const float w0 = wtab[fa * kCF + c];
-        if (!packed) {
+        for (int j = 0; j < 4; ++j) {
+          const int kx = b + 64 * (4 * g + j);
+          const int fa = (kx <= kN / 2) ? kx : kN - kx;
+          const float w0 = wt[fa * kCF + c];
           x[j] = cscale(m[4 * t + j], w0);
-        } else {
-          const float wn = wpk[fa];
-          const float2 dn = DN[(long long)(kx + zo) * kN + ky];  // address rebuilt per radius
-          x[j] = make_float2(w0 * m[4 * t + j].x - wn * dn.y, w0 * m[4 * t + j].y + wn * dn.x);
+          if constexpr (PK) {  // every lane computes it: no branch
+            const float wn = wt[kCF * kNF + fa];
+            const float2 dn = DN[(long long)(kx + zo) * kN + ky];  // address rebuilt per radius
+            const float2 s = make_float2(fmaf(w0, m[4 * t + j].x, -(wn * dn.y)), fmaf(wn, dn.x, w0 * m[4 * t + j].y));
+            x[j] = make_float2(packed ? s.x : x[j].x, packed ? s.y : x[j].y);
+          }
+        }
+        // the filtered values are rounded to FP32 before they are split (no
+        // product contracted into the residual)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) asm("" : "+v"(x[j].x), "+v"(x[j].y));
+        const SplitOp bop = split_b(x);
+        const float4_t d0 = mfma_split(SplitOp{s_gA[0][0][l + zo], s_gA[0][1][l + zo]}, bop);
+        const float4_t d1 = mfma_split(SplitOp{s_gA[1][0][l + zo], s_gA[1][1][l + zo]}, bop);
+        // output q of butterfly b at row 16 b + q
+        const int row = 16 * b + g;
+        bufX[xrow_s(row) * kCF + c] = make_float2(d0[0], d0[1]);
+        bufX[xrow_s(row + 4) * kCF + c] = make_float2(d0[2], d0[3]);
+        bufX[xrow_s(row + 8) * kCF + c] = make_float2(d1[0], d1[1]);
+        bufX[xrow_s(row + 12) * kCF + c] = make_float2(d1[2], d1[3]);
+      }
+      __syncthreads();  // (2) stage A's outputs complete; its W table reads done
+      if (rl + 1 < nb) fill(rl + 1);
+      // stage B: k = w; butterflies b' = w + 16 (2t + sel), inputs at b' + 64 r;
+      // outputs q = g + 4 qi of butterfly t at (2t + sel) 256 + w + 16 q stay in
+      // registers (named values, not an array: no stack copy)
+      float4_t yb[2][2];  // [t][block h]: outputs qi = 2h (d[0], d[1]) and 2h + 1 (d[2], d[3])
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int bp = w + 16 * (2 * t + sel);
+        float2 x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = bufX[xrow_s(bp + 64 * (4 * g + j)) * kCF + c];
+        const SplitOp bop = split_b(x);
+        yb[t][0] = mfma_split(gB0, bop);
+        yb[t][1] = mfma_split(gB1, bop);
+      }
+      // stage C: radix 4, p = 256.  Butterfly b2 = w + 16 (g + 4 qi) takes
+      // inputs r = 2t + sel' from this lane (sel' = sel) and lane l ^ 8; this
+      // lane computes qi = qbase + u (u < 2): block h = sel of its own outputs,
+      // and sends the partner block h = 1 - sel.  The exchange is a DPP row
+      // rotation by 8 (lane l <-> l ^ 8 within each row of 16).
+      float4_t mine[2], recv[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float4_t send;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          mine[t][i] = sel ? yb[t][1][i] : yb[t][0][i];
+          send[i] = sel ? yb[t][0][i] : yb[t][1][i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          recv[t][i] = __int_as_float(
+              __builtin_amdgcn_update_dpp(0, __float_as_int(send[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+      }
+      float2* dst = tp + (long long)rl * plane;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int qi = qbase + u;
+        const int b2 = w + 16 * (g + 4 * qi);
+        const float2 y0 = make_float2(mine[0][2 * u], mine[0][2 * u + 1]);
+        const float2 y1 = make_float2(mine[1][2 * u], mine[1][2 * u + 1]);
+        const float2 p0 = make_float2(recv[0][2 * u], recv[0][2 * u + 1]);
+        const float2 p1 = make_float2(recv[1][2 * u], recv[1][2 * u + 1]);
+        float2 v[4];
+        v[0] = sel ? p0 : y0;
+        v[1] = sel ? y0 : p0;
+        v[2] = sel ? p1 : y1;
+        v[3] = sel ? y1 : p1;
+#pragma unroll
+        for (int r = 1; r < 4; ++r) v[r] = cmul(v[r], s_twc[r * b2 + zo]);
+        DFT<4, +1>::run(v);
+        // Stores of 16 B: lanes c and c ^ 1 (same rows) swap one value, then
+        // the even lane writes columns (c, c + 1) of row q = 2p and the odd lane
+        // columns (c - 1, c) of row 2p + 1.  Same bits as a lane per column;
+        // at 1024^3 x 96 the x pass measured 126.5-129.2 against 130.3-140.9 ms
+        // per step (the y pass after it 2-3 ms slower, the step faster).  The
+        // offsets are rebuilt from the opaque zero each radius (not hoisted out
+        // of the loop and held in registers).
+        const bool odd = (c & 1) != 0;
+        float2* const dste = dst - (odd ? 1 : 0);
+#pragma unroll
+        for (int pp = 0; pp < 2; ++pp) {
+          const float2 a = cscale(v[2 * pp], ibs), bq = cscale(v[2 * pp + 1], ibs);
+          const float2 snd = odd ? a : bq;
+          const float2 rcv = make_float2(
+              __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(snd.x), 0xB1 /* quad_perm [1,0,3,2] */, 0xf, 0xf,
+                                                      false)),
+              __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(snd.y), 0xB1, 0xf, 0xf, false)));
+          const float4 o = odd ? make_float4(rcv.x, rcv.y, bq.x, bq.y) : make_float4(a.x, a.y, rcv.x, rcv.y);
+          const long long row = b2 + zo + 256 * (2 * pp + (odd ? 1 : 0));
+          *reinterpret_cast<float4*>(dste + row * kN * kC) = o;
         }
       }
-      const SplitOp bop = split_b(x);
-      const float4_t d0 = mfma_split(SplitOp{s_gA[0][0][l + zo], s_gA[0][1][l + zo]}, bop);
-      const float4_t d1 = mfma_split(SplitOp{s_gA[1][0][l + zo], s_gA[1][1][l + zo]}, bop);
-      // output q of butterfly b at row 16 b + q
-      const int row = 16 * b + g;
-      bufX[xrow_s(row) * kCF + c] = make_float2(d0[0], d0[1]);
-      bufX[xrow_s(row + 4) * kCF + c] = make_float2(d0[2], d0[3]);
-      bufX[xrow_s(row + 8) * kCF + c] = make_float2(d1[0], d1[1]);
-      bufX[xrow_s(row + 12) * kCF + c] = make_float2(d1[2], d1[3]);
     }
-    __syncthreads();  // (2) stage A's outputs complete; its W table reads done
-    // stage B: k = w; butterflies b' = w + 16 (2t + sel), inputs at b' + 64 r;
-    // outputs q = g + 4 qi of butterfly t at (2t + sel) 256 + w + 16 q stay in
-    // registers (named values, not an array: no stack copy)
-    float4_t yb[2][2];  // [t][block h]: outputs qi = 2h (d[0], d[1]) and 2h + 1 (d[2], d[3])
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int bp = w + 16 * (2 * t + sel);
-      float2 x[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = bufX[xrow_s(bp + 64 * (4 * g + j)) * kCF + c];
-      const SplitOp bop = split_b(x);
-      yb[t][0] = mfma_split(gB0, bop);
-      yb[t][1] = mfma_split(gB1, bop);
-    }
-    // stage C: radix 4, p = 256.  Butterfly b2 = w + 16 (g + 4 qi) takes
-    // inputs r = 2t + sel' from this lane (sel' = sel) and lane l ^ 8; this
-    // lane computes qi = qbase + u (u < 2): block h = sel of its own outputs,
-    // and sends the partner block h = 1 - sel.  The exchange is a DPP row
-    // rotation by 8 (lane l <-> l ^ 8 within each row of 16).
-    float4_t mine[2], recv[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float4_t send;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        mine[t][i] = sel ? yb[t][1][i] : yb[t][0][i];
-        send[i] = sel ? yb[t][0][i] : yb[t][1][i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        recv[t][i] = __int_as_float(
-            __builtin_amdgcn_update_dpp(0, __float_as_int(send[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
-    }
-    float2* dst = tp + (long long)rl * plane;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int qi = qbase + u;
-      const int b2 = w + 16 * (g + 4 * qi);
-      const float2 y0 = make_float2(mine[0][2 * u], mine[0][2 * u + 1]);
-      const float2 y1 = make_float2(mine[1][2 * u], mine[1][2 * u + 1]);
-      const float2 p0 = make_float2(recv[0][2 * u], recv[0][2 * u + 1]);
-      const float2 p1 = make_float2(recv[1][2 * u], recv[1][2 * u + 1]);
-      float2 v[4];
-      v[0] = sel ? p0 : y0;
-      v[1] = sel ? y0 : p0;
-      v[2] = sel ? p1 : y1;
-      v[3] = sel ? y1 : p1;
-#pragma unroll
-      for (int r = 1; r < 4; ++r) v[r] = cmul(v[r], s_twc[r * b2 + zo]);
-      DFT<4, +1>::run(v);
-      // Stores of 16 B: lanes c and c ^ 1 (same rows) swap one value, then
-      // the even lane writes columns (c, c + 1) of row q = 2p and the odd lane
-      // columns (c - 1, c) of row 2p + 1.  Same bits as a lane per column;
-      // at 1024^3 x 96 the x pass measured 126.5-129.2 against 130.3-140.9 ms
-      // per step (the y pass after it 2-3 ms slower, the step faster).  The
-      // offsets are rebuilt from the opaque zero each radius (not hoisted out
-      // of the loop and held in registers).
-      const bool odd = (c & 1) != 0;
-      float2* const dste = dst - (odd ? 1 : 0);
-#pragma unroll
-      for (int pp = 0; pp < 2; ++pp) {
-        const float2 a = cscale(v[2 * pp], ibs), bq = cscale(v[2 * pp + 1], ibs);
-        const float2 snd = odd ? a : bq;
-        const float2 rcv = make_float2(
-            __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(snd.x), 0xB1 /* quad_perm [1,0,3,2] */, 0xf, 0xf,
-                                                    false)),
-            __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(snd.y), 0xB1, 0xf, 0xf, false)));
-        const float4 o = odd ? make_float4(rcv.x, rcv.y, bq.x, bq.y) : make_float4(a.x, a.y, rcv.x, rcv.y);
-        const long long row = b2 + zo + 256 * (2 * pp + (odd ? 1 : 0));
-        *reinterpret_cast<float4*>(dste + row * kN * kC) = o;
-      }
-    }
-  }
+  };
+  if (has_packed) radii(std::true_type{});
+  else radii(std::false_type{});
 }
 
 // ---------------------------------------------------------------- z pass
