@@ -548,15 +548,28 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
     for (int e = 0; e < E; ++e) {
       const int kx = i + e * T;
       const int fa = (kx <= N / 2) ? kx : N - kx;
-      const float w0 = wtab[fa * CF + cl];
-      if (!packed) {
-        v[e] = cscale(m[e], w0);
-      } else {
-        const float wn = wpk[fa];
+      v[e] = cscale(m[e], wtab[fa * CF + cl]);
+    }
+    // Block-uniform, then every lane computes it and column 0 keeps it: a branch
+    // per value, taken by one lane in CF, made each value wait for its own LDS
+    // read.  x pass at 128^3 x 32: 91 -> 86 us, 192^3 x 24: 255 -> 238, 256^3 x 48:
+    // 795 -> 645, 512^3 x 64: 7.97 -> 7.6 ms (FP16 7.71 -> 6.9), 1024^3 x 32: 38.3
+    // -> 37.0 ms.
+    if (has_packed) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int kx = i + e * T;
+        const int fa = (kx <= N / 2) ? kx : N - kx;
+        const float w0 = wtab[fa * CF + cl], wn = wpk[fa];
         const float2 b = DN[(long long)kx * N + ky];
-        v[e] = make_float2(w0 * m[e].x - wn * b.y, w0 * m[e].y + wn * b.x);
+        const float2 s = make_float2(fmaf(w0, m[e].x, -(wn * b.y)), fmaf(w0, m[e].y, wn * b.x));
+        v[e] = make_float2(packed ? s.x : v[e].x, packed ? s.y : v[e].y);
       }
     }
+    // the filtered values are rounded before the transform (no product
+    // contracted into its first additions)
+#pragma unroll
+    for (int e = 0; e < E; ++e) asm("" : "+v"(v[e].x), "+v"(v[e].y));
     auto next = [&] {
       if (rl + 1 < nb) fill(rl + 1);
     };
