@@ -541,13 +541,16 @@ __global__ void __launch_bounds__(kFzThreads) __attribute__((amdgpu_waves_per_eu
     // zreion (and rbubble) of row base + w, element pair n = l + 64 m (+ 256)
     float2* zp = reinterpret_cast<float2*>(zre + (base + w) * kN);
     float2* bp2 = RB ? reinterpret_cast<float2*>(rbub + (base + w) * kN) : nullptr;
+    // all loads before the first store, behind which each would wait in turn
+    float2 old[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) old[e] = zp[l + 64 * (e & 3) + 256 * (e >> 2)];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int nn = l + 64 * (e & 3) + 256 * (e >> 2);
-      const float2 old = zp[nn];
-      const bool u0 = best[e].x > old.x, u1 = best[e].y > old.y;
+      const bool u0 = best[e].x > old[e].x, u1 = best[e].y > old[e].y;
       if (u0 || u1) {
-        zp[nn] = make_float2(u0 ? best[e].x : old.x, u1 ? best[e].y : old.y);
+        zp[nn] = make_float2(u0 ? best[e].x : old[e].x, u1 ? best[e].y : old[e].y);
         if (RB) {
           const float2 ob = bp2[nn];
           bp2[nn] = make_float2(u0 ? bR0[e] : ob.x, u1 ? bR1[e] : ob.y);
