@@ -34,12 +34,23 @@ struct Blk {
 // apart by a multiple of SW share their permutation, and any 64 rows from a
 // multiple of 64 on stay consecutive.  FP16 planes and smaller grids, which the
 // Infinity Cache holds in part, gained nothing from it.
+//
+// The FP16 planes of N = 1024 pair neighbouring x instead (kPair): an x block has 8
+// of the 16 columns, 32 B of each row, and the row of (x, y, half s of the columns)
+// is stored as half x mod 2 of row y of plane (x - x mod 2) + s, so that two lanes
+// groups' pieces make one of 64 B.  A y tile transforms its 16 columns alike
+// whatever they are; a z block takes rows of both x and reads whole lines.
 template <int N, class TS>
 struct TLay {
   static constexpr bool kOn = N >= 512 && sizeof(TS) == 8;
   static constexpr int SW = !kOn ? 1 : (N == 512 ? 8 : 16);
   static constexpr int SH = !kOn ? 0 : (N == 2048 ? 7 : 6);
   static __device__ __forceinline__ int swap(int x) { return (x & (SW - 1)) << SH; }
+  static constexpr bool kPair = N == 1024 && sizeof(TS) == 4;
+  // where column c of plane x is stored, as an offset in values from its plain place
+  static __device__ __forceinline__ int shift(int x, int c) {
+    return kPair ? ((c >> 3) - (x & 1)) * (N * Blk<N>::C) + 8 * (x & 1) + (c & 7) - c : 0;
+  }
   // stored row index of z row r = x N + y
   static __device__ __forceinline__ long long row(long long r) { return kOn ? r ^ swap((int)(r / N)) : r; }
 };

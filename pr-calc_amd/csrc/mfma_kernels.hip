@@ -23,6 +23,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "d2z_device.h"
 #include "d2z_kernels.h"
 #include "fft_core.h"
@@ -103,6 +105,13 @@ constexpr int kMatSets = 2 + 2 * 16;
 __device__ __forceinline__ int mat_set_a(int h) { return h; }
 __device__ __forceinline__ int mat_set_b(int k, int h) { return 2 + 2 * k + h; }
 
+// Ends the wait for the spectrum loads here: inside the radius loop it would be a
+// wait for the stores of the radius before, which the same counter counts.
+__device__ __forceinline__ void pin_loads(float2 (&m)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) asm volatile("" : "+v"(m[k].x), "+v"(m[k].y));
+}
+
 __global__ void __launch_bounds__(64) k_mfma_mats(half8_t* __restrict__ out) {
   const int set = blockIdx.x, l = threadIdx.x;
   out[set * 64 + l] = set < 2 ? stage_matrix(0, 1, set, l) : stage_matrix((set - 2) >> 1, 16, (set - 2) & 1, l);
@@ -117,10 +126,9 @@ __global__ void __launch_bounds__(kThreads)
   constexpr long long plane = (long long)kN * kN * Nh;
   __shared__ uint32_t bufX[kN * kCF];
   __shared__ uint32_t bufY[kN * kCF];
-  __shared__ float wtab[(kCF + 1) * kNF];  // [|fx|][column], then the kz = N/2 column
-  __shared__ float ktab[(kCF + 1) * kNF];  // |k|/dk of the same entries
-  extern __shared__ float4 wsh[];           // W(x) interpolation table (wM intervals)
-  float* wpk = wtab + kCF * kNF;
+  constexpr int kWT = (kCF + 1) * kNF;
+  __shared__ float wtab[2][kWT];   // of two radii: [|fx|][column], then the kz = N/2 column
+  extern __shared__ float4 wsh[];  // W(x) interpolation table (wM intervals)
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
@@ -152,88 +160,94 @@ __global__ void __launch_bounds__(kThreads)
     }
   }
   const int fy2 = fsq(ky, kN);
-  const int ntab = (has_packed ? kCF + 1 : kCF) * kNF;
-  for (int q = tid; q < ntab; q += kThreads) {
-    int f, kzq;
-    if (q < kCF * kNF) {
-      f = q / kCF;
-      kzq = kz0 + q % kCF;
-    } else {
-      f = q - kCF * kNF;
-      kzq = kN / 2;
-    }
-    ktab[q] = kmag_grid(f * f + fy2 + kzq * kzq);
-  }
   for (int q = tid; q < wM; q += kThreads) wsh[q] = wcoef[q];
   // stage-C thread layout: column cl, butterflies i and i + 128
   const int cl = tid & 7, ic = tid >> 3;
-  __half2* tp = Tbuf + (long long)kzb * kN * kN * kC + (long long)ky * kC + sub * kCF + cl;
+  using TL = TLay<kN, __half2>;
+  static_assert(TL::kPair, "the x pass stores x = ic + 128 n, paired by ic");
+  __half2* tp = Tbuf + (long long)kzb * kN * kN * kC + (long long)ky * kC + sub * kCF + cl +
+                TL::shift(ic, sub * kCF + cl);
+  pin_loads(m);
   __syncthreads();
 
+  // The W table is double-buffered: the next radius's is filled between the two
+  // barriers of a radius, beside stage B.  Blocks without the packed column
+  // take a loop without it: a branch per value made each wait for its own LDS
+  // read, and the first use of the spectrum loads inside the loop waited for
+  // the stores of the radius before.  1024^3 x 32: 32.2-33.1 -> 27.6-27.8 ms with
+  // the paired planes; either alone measured 30.5-34.8.
+  auto radii = [&](auto pk) {
+    constexpr bool PK = decltype(pk)::value;
+    auto fill = [&](int rl) {
+      const float dkR = dk * rc[r0 + rl].R;
+      fill_wcolumns<kN, kCF, kThreads, PK>(wtab[rl & 1], fy2, kz0, dkR, dkR * winvh, invN3, wsh, wM, tid);
+    };
+    fill(0);
+    __syncthreads();
 #pragma unroll 1
-  for (int rl = 0; rl < nb; ++rl) {
-    const float dkR = dk * rc[r0 + rl].R;
-    const float dkRh = dkR * winvh;
-    // (the unrolled fill_wtable measured slower here: it pushes this kernel
-    // from 8 to 20 bytes of spills)
-    for (int q = tid; q < ntab; q += kThreads) wtab[q] = filter_from_table(ktab[q], dkR, dkRh, invN3, wsh, wM);
-    __syncthreads();
-    // stage A: filter, radix 16 on the matrix cores, outputs to bufX
+    for (int rl = 0; rl < nb; ++rl) {
+      int zo = 0;  // opaque zero: the packed column's addresses are rebuilt per radius
+      if constexpr (PK) asm volatile("" : "+v"(zo));
+      const float* wt = wtab[rl & 1];
+      // stage A: filter, radix 16 on the matrix cores, outputs to bufX
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int b = 4 * w + 2 * t + sel;
-      float2 x[4];
+      for (int t = 0; t < 2; ++t) {
+        const int b = 4 * w + 2 * t + sel;
+        float2 x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int kx = b + 64 * (4 * g + j);
-        const int fa = (kx <= kN / 2) ? kx : kN - kx;
-        const float w0 = wtab[fa * kCF + c];
-        if (!packed) {
+        for (int j = 0; j < 4; ++j) {
+          const int kx = b + 64 * (4 * g + j);
+          const int fa = (kx <= kN / 2) ? kx : kN - kx;
+          const float w0 = wt[fa * kCF + c];
           x[j] = cscale(m[4 * t + j], w0);
-        } else {
-          const float wn = wpk[fa];
-          const float2 dn = DN[(long long)kx * kN + ky];
-          x[j] = make_float2(w0 * m[4 * t + j].x - wn * dn.y, w0 * m[4 * t + j].y + wn * dn.x);
+          if constexpr (PK) {  // every lane computes it: no branch
+            const float wn = wt[kCF * kNF + fa];
+            const float2 dn = DN[(long long)(kx + zo) * kN + ky];
+            const float2 s = make_float2(fmaf(w0, m[4 * t + j].x, -(wn * dn.y)), fmaf(wn, dn.x, w0 * m[4 * t + j].y));
+            x[j] = make_float2(packed ? s.x : x[j].x, packed ? s.y : x[j].y);
+          }
         }
+        const half8_t bop = pack_b(x);
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+        const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA0, bop, z, 0, 0, 0);
+        const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA1, bop, z, 0, 0, 0);
+        // output q of butterfly b at 16 b + q
+        store_d(bufX, d0, d1, 16 * b + g, 1, c);
       }
-      const half8_t bop = pack_b(x);
-      const float4_t z = {0.f, 0.f, 0.f, 0.f};
-      const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA0, bop, z, 0, 0, 0);
-      const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA1, bop, z, 0, 0, 0);
-      // output q of butterfly b at 16 b + q
-      store_d(bufX, d0, d1, 16 * b + g, 1, c);
+      __syncthreads();  // stage A's outputs complete; the last radius's bufY reads done
+      if (rl + 1 < nb) fill(rl + 1);
+      // stage B: k = w; butterflies b' = w + 16 (2t + sel), inputs at b' + 64 r
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int bp = w + 16 * (2 * t + sel);
+        const half8_t bop = load_b(bufX, bp + 64 * 4 * g, 64, c);
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+        const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB0, bop, z, 0, 0, 0);
+        const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB1, bop, z, 0, 0, 0);
+        // output q at (b' / 16) 256 + k + 16 q
+        store_d(bufY, d0, d1, (bp >> 4) * 256 + w + 16 * g, 16, c);
+      }
+      __syncthreads();  // stage B's outputs and the next W table complete
+      // stage C: radix 4, p = 256, twiddles w1024^(r b''), natural-order outputs
+      __half2* dst = tp + (long long)rl * plane;
+#pragma unroll
+      for (int mm = 0; mm < 2; ++mm) {
+        const int b2 = ic + 128 * mm;
+        float2 u[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[r] = unpack_h2(bufY[xrow(b2 + 256 * r) * kCF + cl]);
+#pragma unroll
+        for (int r = 1; r < 4; ++r) u[r] = cmul(u[r], tw_full[256 + 4 * b2 + r]);
+        DFT<4, +1>::run(u);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dst[(long long)(b2 + 256 * q) * kN * kC] = __float22half2_rn(u[q]);
+      }
+      // next radius: stage A writes bufX, whose stage-B reads end at the barrier
+      // above; its fill writes the W table that this radius's stage A read
     }
-    __syncthreads();
-    // stage B: k = w; butterflies b' = w + 16 (2t + sel), inputs at b' + 64 r
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int bp = w + 16 * (2 * t + sel);
-      const half8_t bop = load_b(bufX, bp + 64 * 4 * g, 64, c);
-      const float4_t z = {0.f, 0.f, 0.f, 0.f};
-      const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB0, bop, z, 0, 0, 0);
-      const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB1, bop, z, 0, 0, 0);
-      // output q at (b' / 16) 256 + k + 16 q
-      store_d(bufY, d0, d1, (bp >> 4) * 256 + w + 16 * g, 16, c);
-    }
-    __syncthreads();
-    // stage C: radix 4, p = 256, twiddles w1024^(r b''), natural-order outputs
-    __half2* dst = tp + (long long)rl * plane;
-#pragma unroll
-    for (int mm = 0; mm < 2; ++mm) {
-      const int b2 = ic + 128 * mm;
-      float2 u[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = unpack_h2(bufY[xrow(b2 + 256 * r) * kCF + cl]);
-#pragma unroll
-      for (int r = 1; r < 4; ++r) u[r] = cmul(u[r], tw_full[256 + 4 * b2 + r]);
-      DFT<4, +1>::run(u);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) dst[(long long)(b2 + 256 * q) * kN * kC] = __float22half2_rn(u[q]);
-    }
-    // next radius: wtab was last read in stage A and bufX in stage B, both
-    // before a barrier; bufY (read just above) is rewritten in stage B only
-    // after the barriers that follow the table fill and stage A
-  }
+  };
+  if (has_packed) radii(std::true_type{});
+  else radii(std::false_type{});
 }
 
 // ------------------------------------------------------ x pass, N = 2048
@@ -279,9 +293,9 @@ __global__ void __launch_bounds__(x2048::kThreads)
   constexpr long long plane = (long long)N2 * N2 * (N2 / 2);
   __shared__ uint32_t bufX[N2 * CF2];
   __shared__ uint32_t bufY[N2 * CF2];
-  __shared__ float wtab[(CF2 + 1) * NF2];  // [|fx|][column], then the kz = N/2 column
-  extern __shared__ float4 wsh[];           // W(x) interpolation table (wM intervals)
-  float* wpk = wtab + CF2 * NF2;
+  constexpr int kWT2 = (CF2 + 1) * NF2;
+  __shared__ float wtab[2][kWT2];  // of two radii: [|fx|][column], then the kz = N/2 column
+  extern __shared__ float4 wsh[];  // W(x) interpolation table (wM intervals)
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
@@ -310,104 +324,101 @@ __global__ void __launch_bounds__(x2048::kThreads)
     }
   }
   const int fy2 = fsq(ky, N2);
-  const int ntab = (has_packed ? CF2 + 1 : CF2) * NF2;
   for (int q = tid; q < wM; q += T2) wsh[q] = wcoef[q];
   const int cl = tid & 3, b2 = tid >> 2;  // stage C: column cl, butterfly b2 < 256
   __half2* tp = Tbuf + (long long)kzb * N2 * N2 * C2 + (long long)ky * C2 + sub * CF2 + cl;
+  pin_loads(m);
   __syncthreads();
 
+  auto radii = [&](auto pk) {
+    constexpr bool PK = decltype(pk)::value;
+    auto fill = [&](int rl) {
+      const float dkR = dk * rc[r0 + rl].R;
+      fill_wcolumns<N2, CF2, T2, PK>(wtab[rl & 1], fy2, kz0, dkR, dkR * winvh, invN3, wsh, wM, tid);
+    };
+    fill(0);
+    __syncthreads();
 #pragma unroll 1
-  for (int rl = 0; rl < nb; ++rl) {
-    // opaque zero: the radius-invariant LDS and store addresses and the
-    // stage-C twiddles are rebuilt per radius instead of held in registers
-    int zo = 0;
-    asm volatile("" : "+v"(zo));
-    const float dkR = dk * rc[r0 + rl].R;
-    const float dkRh = dkR * winvh;
-    for (int q = tid; q < ntab; q += T2) {
-      int f, kzq;
-      if (q < CF2 * NF2) {
-        f = q / CF2;
-        kzq = kz0 + q % CF2;
-      } else {
-        f = q - CF2 * NF2;
-        kzq = N2 / 2;
-      }
-      wtab[q] = filter_from_table(kmag_grid(f * f + fy2 + kzq * kzq), dkR, dkRh, invN3, wsh, wM);
-    }
-    __syncthreads();  // (1) W table complete; bufX's stage-B reads of the last radius done
-    // stage A: filter, radix 16 on the matrix cores, outputs to bufX
+    for (int rl = 0; rl < nb; ++rl) {
+      const float* wt = wtab[rl & 1];
+      // opaque zero: the radius-invariant LDS and store addresses and the
+      // stage-C twiddles are rebuilt per radius instead of held in registers
+      int zo = 0;
+      asm volatile("" : "+v"(zo));
+      // stage A: filter, radix 16 on the matrix cores, outputs to bufX
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int b = 8 * w + 4 * t + sel;
-      float2 x[4];
+      for (int t = 0; t < 2; ++t) {
+        const int b = 8 * w + 4 * t + sel;
+        float2 x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int kx = b + 128 * (4 * g + j);
-        const int fa = (kx <= N2 / 2) ? kx : N2 - kx;
-        const float w0 = wtab[fa * CF2 + c];
-        if (!packed) {
+        for (int j = 0; j < 4; ++j) {
+          const int kx = b + 128 * (4 * g + j);
+          const int fa = (kx <= N2 / 2) ? kx : N2 - kx;
+          const float w0 = wt[fa * CF2 + c];
           x[j] = cscale(m[4 * t + j], w0);
-        } else {
-          const float wn = wpk[fa];
-          const float2 dn = DN[(long long)kx * N2 + ky];
-          x[j] = make_float2(w0 * m[4 * t + j].x - wn * dn.y, w0 * m[4 * t + j].y + wn * dn.x);
+          if constexpr (PK) {  // every lane computes it: no branch
+            const float wn = wt[CF2 * NF2 + fa];
+            const float2 dn = DN[(long long)(kx + zo) * N2 + ky];
+            const float2 s = make_float2(fmaf(w0, m[4 * t + j].x, -(wn * dn.y)), fmaf(wn, dn.x, w0 * m[4 * t + j].y));
+            x[j] = make_float2(packed ? s.x : x[j].x, packed ? s.y : x[j].y);
+          }
         }
+        const half8_t bop = pack_b(x);
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+        const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA0, bop, z, 0, 0, 0);
+        const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA1, bop, z, 0, 0, 0);
+        // outputs q = g, g + 4 (block 0), g + 8, g + 12 (block 1) at 16 b + q
+        const int row = 16 * b + g + zo;
+        bufX[xsw(row) * CF2 + c] = pack_h2(d0[0], d0[1]);
+        bufX[xsw(row + 4) * CF2 + c] = pack_h2(d0[2], d0[3]);
+        bufX[xsw(row + 8) * CF2 + c] = pack_h2(d1[0], d1[1]);
+        bufX[xsw(row + 12) * CF2 + c] = pack_h2(d1[2], d1[3]);
       }
-      const half8_t bop = pack_b(x);
-      const float4_t z = {0.f, 0.f, 0.f, 0.f};
-      const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA0, bop, z, 0, 0, 0);
-      const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gA1, bop, z, 0, 0, 0);
-      // outputs q = g, g + 4 (block 0), g + 8, g + 12 (block 1) at 16 b + q
-      const int row = 16 * b + g + zo;
-      bufX[xsw(row) * CF2 + c] = pack_h2(d0[0], d0[1]);
-      bufX[xsw(row + 4) * CF2 + c] = pack_h2(d0[2], d0[3]);
-      bufX[xsw(row + 8) * CF2 + c] = pack_h2(d1[0], d1[1]);
-      bufX[xsw(row + 12) * CF2 + c] = pack_h2(d1[2], d1[3]);
+      __syncthreads();  // stage A's outputs complete; the last radius's bufY reads done
+      if (rl + 1 < nb) fill(rl + 1);
+      // stage B: k = w; butterflies b' = w + 16 (4 t + sel), inputs at b' + 128 r
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int bp = w + 16 * (4 * t + sel);
+        union {
+          uint32_t u[4];
+          half8_t h;
+        } cv;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cv.u[j] = bufX[xsw(bp + zo + 128 * (4 * g + j)) * CF2 + c];
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+        const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB0, cv.h, z, 0, 0, 0);
+        const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB1, cv.h, z, 0, 0, 0);
+        // output q at 256 (b' / 16) + w + 16 q
+        const int row = (bp >> 4) * 256 + w + 16 * g + zo;
+        bufY[ysw(row) * CF2 + c] = pack_h2(d0[0], d0[1]);
+        bufY[ysw(row + 64) * CF2 + c] = pack_h2(d0[2], d0[3]);
+        bufY[ysw(row + 128) * CF2 + c] = pack_h2(d1[0], d1[1]);
+        bufY[ysw(row + 192) * CF2 + c] = pack_h2(d1[2], d1[3]);
+      }
+      __syncthreads();  // stage B's outputs and the next W table complete
+      // stage C: radix 8, p = 256, natural-order outputs
+      __half2* dst = tp + (long long)rl * plane;
+      float2 u[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) u[r] = unpack_h2(bufY[ysw(b2 + zo + 256 * r) * CF2 + cl]);
+#pragma unroll
+      for (int r = 1; r < 8; ++r) u[r] = cmul(u[r], tw_plan[256 + 8 * b2 + r + zo]);
+      DFT<8, +1>::run(u);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) dst[(long long)(b2 + zo + 256 * q) * N2 * C2] = __float22half2_rn(u[q]);
+      // the next radius: as in k_fx_mfma
     }
-    __syncthreads();  // (2) stage A's outputs complete
-    // stage B: k = w; butterflies b' = w + 16 (4 t + sel), inputs at b' + 128 r
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int bp = w + 16 * (4 * t + sel);
-      union {
-        uint32_t u[4];
-        half8_t h;
-      } cv;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) cv.u[j] = bufX[xsw(bp + zo + 128 * (4 * g + j)) * CF2 + c];
-      const float4_t z = {0.f, 0.f, 0.f, 0.f};
-      const float4_t d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB0, cv.h, z, 0, 0, 0);
-      const float4_t d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gB1, cv.h, z, 0, 0, 0);
-      // output q at 256 (b' / 16) + w + 16 q
-      const int row = (bp >> 4) * 256 + w + 16 * g + zo;
-      bufY[ysw(row) * CF2 + c] = pack_h2(d0[0], d0[1]);
-      bufY[ysw(row + 64) * CF2 + c] = pack_h2(d0[2], d0[3]);
-      bufY[ysw(row + 128) * CF2 + c] = pack_h2(d1[0], d1[1]);
-      bufY[ysw(row + 192) * CF2 + c] = pack_h2(d1[2], d1[3]);
-    }
-    __syncthreads();  // (3) stage B's outputs complete
-    // stage C: radix 8, p = 256, natural-order outputs
-    __half2* dst = tp + (long long)rl * plane;
-    float2 u[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) u[r] = unpack_h2(bufY[ysw(b2 + zo + 256 * r) * CF2 + cl]);
-#pragma unroll
-    for (int r = 1; r < 8; ++r) u[r] = cmul(u[r], tw_plan[256 + 8 * b2 + r + zo]);
-    DFT<8, +1>::run(u);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) dst[(long long)(b2 + zo + 256 * q) * N2 * C2] = __float22half2_rn(u[q]);
-    // next radius: wtab was last read in stage A and bufX in stage B, both
-    // before a barrier; bufY (read just above) is rewritten in stage B only
-    // after the barriers that follow the table fill and stage A
-  }
+  };
+  if (has_packed) radii(std::true_type{});
+  else radii(std::false_type{});
 }
 
 // ---------------------------------------------------------------- z pass
-// Last inverse pass (z, c2r) of the mixed path at N = 1024 with the barrier
+// Last inverse pass (z, c2r) of the half path at N = 1024 with the barrier
 // fused, as k_fz (reference delta2zreion_d2z.C:92-146,206-216), for blocks of
-// 8 consecutive z rows (512 B contiguous per kz block in the T layout).  Per
-// radius: the raw FP16 rows are staged in LDS; stage A forms the complex
+// 8 z rows, 4 values of y of 2 of x (256 B contiguous per 8 kz in the paired T
+// layout).  Per radius: the raw FP16 rows are staged in LDS; stage A forms the complex
 // sequence Z[k] of the half-length c2r from X[k] and X[L-k] (packed FP16) and
 // runs radix 16 on the matrix cores; stage B (radix 16, p = 16) groups the 16
 // butterflies {k, k+16} x 8 rows that share k = b mod 16; stage C (radix 2,
@@ -466,17 +477,26 @@ __global__ void __launch_bounds__(512)
     s_gB[w][t][1][l] = mats[mat_set_b(2 * w + t, 1) * 64 + l];
   }
   const double sc = (double)iscale, sc2 = sc * sc;
-  // raw-load mapping: each half wave one row: kz = 16 kzb + (t & 15) with
-  // kzb = ((t >> 4) & 1) + 2 (t >> 8) + 4 e, row (t >> 5) & 7
-  const int lrow = (tid >> 5) & 7, lkz = tid & 15, lkzb = ((tid >> 4) & 1) + 2 * (tid >> 8);
+  // A block's 8 rows are 4 values of y of a pair of x: group G has x = 2 (G / 256)
+  // + row / 4 and y = 4 (G mod 256) + row mod 4 (gridrow).  In the paired layout
+  // (TLay) the 256 B that the four y take in one plane are then columns 8 s .. 8 s
+  // + 7 of all 8 rows, and a wave loads them at once: s = w mod 2, kz block w / 2
+  // + 4 e, lane l at y l / 16, value l mod 16 = 8 (x mod 2) + column.
+  static_assert(TLay<kN, __half2>::kPair && kRowsZ == 8, "rows of a z block");
+  auto gridrow = [](long long base, int row) {
+    const int G = (int)(base / kRowsZ);
+    return (long long)(2 * (G / (kN / 4)) + row / 4) * kN + 4 * (G % (kN / 4)) + row % 4;
+  };
+  const int lraw = zx_at(4 * ((l >> 3) & 1) + (l >> 4), 0) + 8 * w + (l & 7);  // + zx_at(0, 64 e): 8 w + 7 < 64
   const float4_t z4 = {0.f, 0.f, 0.f, 0.f};
   // the raw rows of (group, radius) are loaded into registers one step ahead
   // and stored to LDS at the start of the step, so the loads overlap the
   // previous step's transforms
   uint32_t pf[8];
-  const uint32_t lane_off = ((uint32_t)lkzb * (uint32_t)nrows + (uint32_t)lrow) * 16u + (uint32_t)lkz;
+  const uint32_t lane_off =
+      ((uint32_t)(w >> 1) * (uint32_t)nrows + (uint32_t)((w & 1) * kN + (l >> 4))) * 16u + (uint32_t)(l & 15);
   auto fetch = [&](long long gbase, int q) {
-    const uint32_t* tp = reinterpret_cast<const uint32_t*>(Tbuf + (long long)q * plane + gbase * 16);
+    const uint32_t* tp = reinterpret_cast<const uint32_t*>(Tbuf + (long long)q * plane + gridrow(gbase, 0) * 16);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       // uniform part (kz block 4e) on the scalar base, one per-lane offset
@@ -502,7 +522,7 @@ __global__ void __launch_bounds__(512)
       int zo = 0;  // opaque zero: the matrix reads stay inside the radius loop
       asm volatile("" : "+s"(zo));
 #pragma unroll
-      for (int e = 0; e < 8; ++e) bufX[zx_at(lrow, 16 * (lkzb + 4 * e) + lkz)] = pf[e];
+      for (int e = 0; e < 8; ++e) bufX[lraw + zx_at(0, 64 * e)] = pf[e];
       __syncthreads();
       // stage A: butterflies b = 4w + 2t + sel of row rowA, inputs Z[b + 32 r]
 #pragma unroll
@@ -589,9 +609,10 @@ __global__ void __launch_bounds__(512)
       const double wsum = (double)wave_sum_f(acc) * sc2;
       if (l == 0) red[w][q] += wsum;
     }
-    // zreion (and rbubble) of row base + w, element pair n = l + 64 m (+ 256)
-    float2* zp = reinterpret_cast<float2*>(zre + (base + w) * kN);
-    float2* bp2 = RB ? reinterpret_cast<float2*>(rbub + (base + w) * kN) : nullptr;
+    // zreion (and rbubble) of the block's row w, element pair n = l + 64 m (+ 256)
+    const long long row = gridrow(base, __builtin_amdgcn_readfirstlane(w));
+    float2* zp = reinterpret_cast<float2*>(zre + row * kN);
+    float2* bp2 = RB ? reinterpret_cast<float2*>(rbub + row * kN) : nullptr;
     // all loads before the first store, behind which each would wait in turn
     // (1024^3 x 32: 23.4 -> 23.0 ms)
     float2 old[8];

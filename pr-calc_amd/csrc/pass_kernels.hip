@@ -242,9 +242,11 @@ __global__ void __launch_bounds__(256) k_inv_z(const TS* __restrict__ in, float*
   const long long row = (long long)blockIdx.x * ROWS + rr;
   const bool valid = row < nrows;
   const long long r = TLay<2 * L, TS>::row(valid ? row : 0);
+  static_assert(!TLay<2 * L, TS>::kPair || T % C == 0, "a thread's values share a column");
+  const int shift = TLay<2 * L, TS>::shift((int)(r / (2 * L)), i % C);
   float2 v[E], m[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = ld(in, zrow_offset<P, C>(i, e, r, nrows));
+  for (int e = 0; e < E; ++e) v[e] = ld(in, zrow_offset<P, C>(i, e, r, nrows) + shift);
   mirror_lanes<P>(v, m, i);
   c2r_pre<P>(v, m, i, tw_full);
   pencil_fft<P, +1>(v, i, tw_half, LdsRow<L>{smem + rr * LdsRow<L>::STRIDE});
@@ -511,8 +513,10 @@ __device__ __forceinline__ void fx_body(const float2* __restrict__ S, const floa
   }
   const int fy2 = fsq(ky, N);
   static_assert(T % TLay<N, TS>::SW == 0, "x = i + e*T permutes its rows by i");
+  static_assert(!TLay<N, TS>::kPair || T % 2 == 0, "x is paired by i");
   const int kyt = ky ^ TLay<N, TS>::swap(i);  // stored row of ky in the planes of this thread's x
-  TS* tp = Tbuf + (long long)kzb * N * N * C + (long long)kyt * C + sub * CF + cl;  // element x at tp[x*N*C]
+  TS* tp = Tbuf + (long long)kzb * N * N * C + (long long)kyt * C + sub * CF + cl +
+           TLay<N, TS>::shift(i, sub * CF + cl);  // element x at tp[x*N*C]
   const LdsColPad<SH> lds{smem + cl, CF};
   const int ntab = (has_packed ? CF + 1 : CF) * NF;
   auto kmag = [&](int q) {  // |k|/dk of table entry q
@@ -713,6 +717,8 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
   const long long row = base + rr;
   const bool valid = row < nrows;
   const long long r = TLay<2 * L, TS>::row(valid ? row : 0);
+  static_assert(!TLay<2 * L, TS>::kPair || T % C == 0, "a thread's values share a column");
+  const int shift = TLay<2 * L, TS>::shift((int)(r / (2 * L)), i % C);
   float2 best[E];
   float bR0[E], bR1[E];
 #pragma unroll
@@ -752,7 +758,7 @@ __device__ __forceinline__ void fz_group(const TS* __restrict__ Tbuf, float* __r
       const uint32_t* tu = reinterpret_cast<const uint32_t*>(tp);
       uint32_t a[E], m[E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) a[e] = tu[zrow_offset<P, C>(i, e, r, nrows)];
+      for (int e = 0; e < E; ++e) a[e] = tu[zrow_offset<P, C>(i, e, r, nrows) + shift];
       mirror_lanes<P>(a, m, i);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
