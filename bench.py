@@ -67,7 +67,7 @@ def kernel_alg_bytes(name: str, N: int, nb: int, store_bytes: int) -> float:
                 intermediates (store B/cell each)
     inv_y       reads and writes nb intermediates
     fz_barrier  reads nb intermediates and reads+writes zreion (8 B/cell)
-    plain kernels: filter 8, inv_x/inv_y/inv_z_c2r 8, barrier 12, moments 4 B/cell
+    plain kernels: filter 8, inv_x/inv_y 8, inv_z_barrier 12 B/cell
     """
     cells = float(N) ** 3
     s = float(store_bytes)
@@ -75,7 +75,7 @@ def kernel_alg_bytes(name: str, N: int, nb: int, store_bytes: int) -> float:
         "fx_filter": 4.0 + s * nb,
         "inv_y": 2 * s * nb,
         "fz_barrier": s * nb + 8.0,
-        "filter": 8.0, "inv_x": 8.0, "inv_z_c2r": 8.0, "barrier": 12.0, "moments": 4.0,
+        "filter": 8.0, "inv_x": 8.0, "inv_z_barrier": 12.0,
         "fwd_z_r2c": 8.0, "fwd_y": 8.0, "fwd_x": 8.0,
     }
     return table.get(name, 0.0) * cells

@@ -138,6 +138,10 @@ hipError_t launch_disp(int N, const float2* S, const float2* D0, const float2* D
 constexpr int kPkMaxBins = 512;
 hipError_t launch_pk(int N, const float2* S, const float2* D0, const float2* DN, float dk, float lnkmin, float dlnk,
                      int nk, double pscale, unsigned long long* count, double* sums, hipStream_t s);
+// plain path: launch_inv_z's rows with the barrier of radius r applied and the sum
+// of squares of nblk blocks left in partial[0 .. nblk)
+hipError_t launch_inv_z_barrier(int N, const float2* in, float* zre, float* rbub, const RadiusConst* rc, int r,
+                                double2* partial, int nblk, const float2* twh, const float2* twf, hipStream_t s);
 hipError_t launch_inv_z_h(int N, const void* in, float* out, float iscale, const float2* twh, const float2* twf,
                           hipStream_t s);
 // in-place tiled pass over FP16 intermediates (mixed path), output scaled
@@ -199,9 +203,6 @@ hipError_t launch_mbox(MBPass pass, const MBox* boxes, const long long* first, i
                        int nb, int toff, int maxM, int nblk, int N, bool rb, hipStream_t s);
 
 // element-wise and set-up kernels (d2z_kernels.hip)
-hipError_t launch_barrier(const float* dR, float* zre, float* rbub, long long total, const RadiusConst* rc, int r,
-                          hipStream_t s);
-hipError_t launch_moments(const float* x, long long total, double2* partial, int nblk, hipStream_t s);
 hipError_t launch_moments_finish(const double2* partial, int nblk, int nrad, double invN3, float* sigma_grid_out,
                                  int r0, hipStream_t s);
 hipError_t launch_history(const float* zre, long long total, unsigned int* counts, double dz, int* range,

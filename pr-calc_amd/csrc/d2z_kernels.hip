@@ -27,53 +27,7 @@ __global__ void k_twiddles(float2* __restrict__ tw, int L) {
   }
 }
 
-// plain path: strict running maximum over a real field (delta2zreion_d2z.C:106-146)
-__global__ void k_barrier(const float* __restrict__ dR, float* __restrict__ zre, float* __restrict__ rbub,
-                          long long total, const RadiusConst* __restrict__ rc, int r) {
-  const double A = rc[r].A;
-  const double B = rc[r].B;
-  const float R = rc[r].R;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total;
-       id += (long long)gridDim.x * blockDim.x) {
-    const float z = barrier_z(dR[id], A, B);
-    if (z > zre[id]) {
-      zre[id] = z;
-      if (rbub) rbub[id] = R;
-    }
-  }
-}
-
-// ------------------------------------------ sigma_grid partial sums (plain)
-// Per-block FP64 sums of delta and delta^2 (GetMeanSigma, arrayoperations.C:4-35).
-
-__global__ void __launch_bounds__(256) k_moments(const float* __restrict__ x, long long total,
-                                                 double2* __restrict__ partial) {
-  double s1 = 0.0, s2 = 0.0;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total;
-       id += (long long)gridDim.x * blockDim.x) {
-    const double d = (double)x[id];
-    s1 += d;
-    s2 += d * d;
-  }
-  __shared__ double sh[2][4];
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-  if (l == 0) {
-    sh[0][w] = s1;
-    sh[1][w] = s2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0, b = 0;
-    for (int k = 0; k < (int)(blockDim.x / 64); ++k) {
-      a += sh[0][k];
-      b += sh[1][k];
-    }
-    partial[blockIdx.x] = make_double2(a, b);
-  }
-}
-
+// ------------------------------------------ sigma_grid sums (plain)
 // Fixed-order reduction of per-block partials -> sigma_grid = sqrt(sum d^2 / N^3)
 __global__ void k_moments_finish(const double2* __restrict__ partial, int nblk, int nrad, double invN3,
                                  float* __restrict__ sigma_grid_out, int r0) {
@@ -500,17 +454,6 @@ static inline unsigned grid1(long long n, int bs, long long cap = 1 << 20) {
 
 hipError_t launch_twiddles(float2* tw, int L, hipStream_t s) {
   hipLaunchKernelGGL(k_twiddles, dim3((L + 255) / 256), dim3(256), 0, s, tw, L);
-  return hipGetLastError();
-}
-
-hipError_t launch_barrier(const float* dR, float* zre, float* rbub, long long total, const RadiusConst* rc, int r,
-                          hipStream_t s) {
-  hipLaunchKernelGGL(k_barrier, dim3(grid1(total, 256)), dim3(256), 0, s, dR, zre, rbub, total, rc, r);
-  return hipGetLastError();
-}
-
-hipError_t launch_moments(const float* x, long long total, double2* partial, int nblk, hipStream_t s) {
-  hipLaunchKernelGGL(k_moments, dim3(nblk), dim3(256), 0, s, x, total, partial);
   return hipGetLastError();
 }
 

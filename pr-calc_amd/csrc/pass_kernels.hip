@@ -257,6 +257,70 @@ __global__ void __launch_bounds__(256) k_inv_z(const TS* __restrict__ in, float*
   }
 }
 
+// The plain path's last inverse pass: the same rows as k_inv_z writes, with d2z()
+// per cell (barrier_z, reference delta2zreion_d2z.C:106-146), zreion (and rbubble)
+// raised where it is larger, and one partial sum of delta_R^2 (reference
+// GetMeanSigma, arrayoperations.C:4-35) per block.  delta_R stays in
+// registers: k_inv_z, a pass for the sums and one for the barrier took 27 + 24 + 36
+// us per radius at 256^3, this one 39 (a run of
+// 16 radii 2.63 -> 1.88 ms, 512^3 x 8 12.4 -> 8.6).
+template <class P, int C, bool RB>
+__global__ void __launch_bounds__(256) k_inv_z_barrier(const float2* __restrict__ in, float* __restrict__ zre,
+                                                       float* __restrict__ rbub, long long nrows,
+                                                       const RadiusConst* __restrict__ rc, int rad,
+                                                       double2* __restrict__ partial,
+                                                       const float2* __restrict__ tw_half,
+                                                       const float2* __restrict__ tw_full) {
+  constexpr int L = P::L, T = P::T, E = P::E;
+  constexpr int ROWS = 256 / T;
+  __shared__ float2 smem[ROWS * LdsRow<L>::STRIDE];
+  __shared__ double sh[4];
+  const int t = threadIdx.x;
+  const int i = t % T, rr = t / T;
+  const double A = rc[rad].A, B = rc[rad].B;
+  const float R = rc[rad].R;
+  double s2 = 0.0;
+#pragma unroll 1
+  for (long long base = (long long)blockIdx.x * ROWS; base < nrows; base += (long long)gridDim.x * ROWS) {
+    const long long row = base + rr;
+    const bool valid = row < nrows;
+    const long long r0 = valid ? row : 0, r = TLay<2 * L, float2>::row(r0);
+    float2* zp = reinterpret_cast<float2*>(zre + r0 * (2 * L));
+    float2* bp = RB ? reinterpret_cast<float2*>(rbub + r0 * (2 * L)) : nullptr;
+    float2 v[E], m[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = ld(in, zrow_offset<P, C>(i, e, r, nrows));
+    mirror_lanes<P>(v, m, i);
+    c2r_pre<P>(v, m, i, tw_full);
+    float2 old[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) old[e] = zp[i + e * T];  // in flight during the transform
+    pencil_fft<P, +1>(v, i, tw_half, LdsRow<L>{smem + rr * LdsRow<L>::STRIDE});
+    if (!valid) continue;  // the loop's barriers are in the transform, which every thread runs
+    // the rows end here as they do where they are stored: k_inv_z's bits
+#pragma unroll
+    for (int e = 0; e < E; ++e) asm("" : "+v"(v[e].x), "+v"(v[e].y));
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const float z0 = barrier_z(v[e].x, A, B), z1 = barrier_z(v[e].y, A, B);
+      s2 += (double)v[e].x * (double)v[e].x;
+      s2 += (double)v[e].y * (double)v[e].y;
+      const bool u0 = z0 > old[e].x, u1 = z1 > old[e].y;
+      if (u0 || u1) {
+        zp[i + e * T] = make_float2(u0 ? z0 : old[e].x, u1 ? z1 : old[e].y);
+        if (RB) {
+          const float2 ob = bp[i + e * T];
+          bp[i + e * T] = make_float2(u0 ? R : ob.x, u1 ? R : ob.y);
+        }
+      }
+    }
+  }
+  s2 = wave_sum(s2);
+  if (t % 64 == 0) sh[t / 64] = s2;
+  __syncthreads();
+  if (t == 0) partial[blockIdx.x] = make_double2(0.0, sh[0] + sh[1] + sh[2] + sh[3]);
+}
+
 // ------------------------------------------------- unpack after forward
 // D0(k) = (P(k) + conj P(-k))/2,  DN(k) = -i (P(k) - conj P(-k))/2 with P the
 // packed kz = 0 slot of S; D0/DN indexed [kx][ky].
@@ -1394,6 +1458,19 @@ static hipError_t inv_z_impl(const TS* in, float* out, float iscale, const float
   return hipGetLastError();
 }
 
+template <int N>
+static hipError_t inv_z_barrier_impl(const float2* in, float* zre, float* rbub, const RadiusConst* rc, int r,
+                                     double2* partial, int nblk, const float2* twh, const float2* twf, hipStream_t s) {
+  using P = Plan<N / 2>;
+  constexpr int C = Blk<N>::C;
+  const long long nrows = (long long)N * N;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblk), dim3(256), 0, s, in, zre, rbub, nrows, rc, r, partial, twh, twf);
+    return hipGetLastError();
+  };
+  return rbub ? go(k_inv_z_barrier<P, C, true>) : go(k_inv_z_barrier<P, C, false>);
+}
+
 template <int N, int DIR, class TI, class TO, Axis AX>
 static hipError_t tile_axis(const TI* in, TO* out, const TileMap& mp, float oscale, const float2* tw, hipStream_t s) {
   using P = TilePlan<N>;
@@ -1597,6 +1674,19 @@ hipError_t launch_inv_z(int N, const float2* in, float* out, const float2* twh, 
 #define X(NN) \
   case NN:    \
     return inv_z_impl<NN, float2>(in, out, 1.0f, twh, twf, s);
+    PRC_FOR_EACH_N(X)
+#undef X
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_inv_z_barrier(int N, const float2* in, float* zre, float* rbub, const RadiusConst* rc, int r,
+                                double2* partial, int nblk, const float2* twh, const float2* twf, hipStream_t s) {
+  switch (N) {
+#define X(NN) \
+  case NN:    \
+    return inv_z_barrier_impl<NN>(in, zre, rbub, rc, r, partial, nblk, twh, twf, s);
     PRC_FOR_EACH_N(X)
 #undef X
     default:

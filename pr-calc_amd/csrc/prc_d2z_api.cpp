@@ -240,9 +240,10 @@ float host_dk(const prc_d2z_ctx* c) {
   return (float)(2. * M_PI / (double)box_mpc(c->p));
 }
 
-// Plain path, one radius: separate filter, three inverse passes, moments and
-// barrier.  T1 holds the filtered spectrum (S layout) and then the real field,
-// T2 the intermediate (T layout).
+// Plain path, one radius: separate filter and three inverse passes, the last with
+// the barrier and the sum of squares behind it, or (barrier = false) leaving the
+// real field in T1.  T1 holds the filtered spectrum (S layout), T2 the
+// intermediate (T layout).
 int plain_radius(prc_d2z_ctx* c, int r, bool barrier) {
   const int N = c->N;
   hipStream_t s = c->stream;
@@ -259,21 +260,19 @@ int plain_radius(prc_d2z_ctx* c, int r, bool barrier) {
             "inverse x pass");
   PRC_CHECK(c, timed(c, "inv_y", [&] { return launch_tile(N, +1, T2, T2, ym, c->d_st_full, s); }),
             "inverse y pass");
-  float* dR = reinterpret_cast<float*>(T1);
-  PRC_CHECK(c, timed(c, "inv_z_c2r", [&] {
-              return launch_inv_z(N, T2, dR, c->d_st_half, c->d_tw_full, s);
+  if (!barrier) {
+    PRC_CHECK(c, timed(c, "inv_z_c2r", [&] {
+                return launch_inv_z(N, T2, reinterpret_cast<float*>(T1), c->d_st_half, c->d_tw_full, s);
+              }),
+              "inverse z pass");
+    return PRC_D2Z_OK;
+  }
+  PRC_CHECK(c, timed(c, "inv_z_barrier", [&] {
+              return launch_inv_z_barrier(N, T2, c->d_zre, c->p.RecordBubbleSizes ? c->d_rb : nullptr, c->d_rc, r,
+                                          c->d_mom + (long long)r * kMomentBlocks, kMomentBlocks, c->d_st_half,
+                                          c->d_tw_full, s);
             }),
-            "inverse z pass");
-  if (!barrier) return PRC_D2Z_OK;
-  PRC_CHECK(c, timed(c, "moments", [&] {
-              return launch_moments(dR, c->ncell, c->d_mom + (long long)r * kMomentBlocks, kMomentBlocks, s);
-            }),
-            "moments");
-  PRC_CHECK(c, timed(c, "barrier", [&] {
-              return launch_barrier(dR, c->d_zre, c->p.RecordBubbleSizes ? c->d_rb : nullptr, c->ncell, c->d_rc, r,
-                                    s);
-            }),
-            "barrier");
+            "inverse z pass and barrier");
   return PRC_D2Z_OK;
 }
 
