@@ -79,6 +79,17 @@ __device__ __forceinline__ long long xcd_tile(long long b, long long nblk) {
   return (b % 8) * (nblk / 8) + b / 8;
 }
 
+// The same with XCD j starting 5 j tiles into its range: a y tile is one contiguous
+// power of two of bytes, and without it the XCDs, in step, work on tiles a power of
+// two apart.  Persistent y pass at 1024^3 x 32: FP32 52.0 -> 51.35 ms, FP16 27.9 ->
+// 27.15 (by 37 tiles: 51.3 and 27.7).
+__device__ __forceinline__ long long xcd_tile_staggered(long long b, long long nblk) {
+  const long long m = nblk / 8, tile = xcd_tile(b, nblk);
+  if (nblk % 8 != 0 || m < 64) return tile;
+  const int j = (int)(b % 8);
+  return tile + 5 * j < (j + 1) * m ? tile + 5 * j : tile + 5 * j - m;
+}
+
 // Tile of block b for the x passes, whose tiles are numbered so that each
 // run of `group` consecutive tiles writes whole 128 B lines of the output
 // together (the column parts of a row, and the adjacent rows sharing a line
@@ -89,8 +100,10 @@ __device__ __forceinline__ long long xcd_tile(long long b, long long nblk) {
 // faster than xcd_tile (each XCD on its own range of tiles), same bits: at
 // 1024^3 x 96 the split x pass 122-136 against 137-145 ms per step, the FP32
 // vector x pass 146-162 against 167-169, at 2048^3 x 128 2074 against 2136.
-// The FP16-output x passes measured slower with it (at 1024^3 98-106 against
-// 97-98 ms, at 2048^3 1871 against 1769) and keep xcd_tile.
+// Of the FP16-output x passes the matrix one at 1024^3, whose paired planes need
+// only its two column parts together, takes it with groups of 2 (27.6 -> 26.0 ms per
+// 32 radii; of 4: 27.1-27.9); the others measured slower with it (at 2048^3 1871
+// against 1769 ms) and keep xcd_tile.
 __device__ __forceinline__ long long line_tile(long long b, long long nblk, int group) {
   if (nblk % (8LL * group) != 0) return b;
   const long long slot = b >> 3;

@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(kThreads)
   const int g = l >> 4, n = l & 15;
   const int c = n & 7, sel = n >> 3;  // MFMA column n = (column c, butterfly sel)
 
-  const long long tile = xcd_tile(blockIdx.x, gridDim.x);
+  const long long tile = line_tile(blockIdx.x, gridDim.x, kNSUB);
   const int sub = (int)(tile % kNSUB);
   const int ky = (int)((tile / kNSUB) % kN);
   const int kzb = (int)(tile / (kNSUB * kN));

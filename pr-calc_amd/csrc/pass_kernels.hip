@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(P::T* C)
 }
 
 // Persistent in-place tile pass (the y passes; TS = float2 or __half2 storage):
-// block b walks tiles vb = b + k gridDim.x (through the same XCD-aware map) and
+// block b walks tiles vb = b + k gridDim.x (through xcd_tile_staggered) and
 // loads tile vb + gridDim.x into registers, in the storage type, while tile vb
 // is transformed and stored, so one tile's loads overlap the previous tile's
 // arithmetic.  pencil_fft ends with a barrier after its last LDS read, so the
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(P::T* C)
   const long long lane_off = c + (long long)i * sA;
   using TL = TLay<L, TS>;
   auto tile_base = [&](long long vb, int& perm) {
-    const long long tile = xcd_tile(vb, ntiles);
+    const long long tile = xcd_tile_staggered(vb, ntiles);
     perm = (int)(tile % nOuter) & (TL::SW - 1);  // the plane's row permutation: see tile_body
     return (tile / nOuter) * sCB + (tile % nOuter) * sO + lane_off;
   };

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 def test_rows_and_sums(N, rbub):
     announce(f"plain z pass N={N} rbubble={rbub}")
     f = field(N)
-    lp = lib_params(N, nscales=5, mode=PLAIN_FP32, rbubble=rbub)
+    lp = lib_params(N, nscales=5, mode=PLAIN_FP32, rbub=rbub)
     with D2Z(lp) as d:
         d.set_delta(f)
         d.run()
@@ -30,4 +30,5 @@ def test_rows_and_sums(N, rbub):
     assert zreion_metrics(z, zo)["max_abs"] <= 2e-4
     if rbub:
         assert np.array_equal(rb > 0, z > 0)
-        assert set(np.unique(rb[rb > 0])) <= set(table[:, 0].astype(np.float32))
+        # recorded in Mpc, the table's first column in Mpc/h
+        assert all(np.isclose(R * lp.h, table[:, 0], rtol=1e-6).any() for R in np.unique(rb[rb > 0]))
