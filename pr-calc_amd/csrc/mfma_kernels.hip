@@ -129,6 +129,7 @@ __global__ void __launch_bounds__(kThreads)
   constexpr int kWT = (kCF + 1) * kNF;
   __shared__ float wtab[2][kWT];   // of two radii: [|fx|][column], then the kz = N/2 column
   extern __shared__ float4 wsh[];  // W(x) interpolation table (wM intervals)
+  static_assert((2 * kN * kCF + 2 * kWT) * 4 + 16 * kWTableMax <= 160 * 1024, "LDS with the longest W(x) table");
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
@@ -170,8 +171,9 @@ __global__ void __launch_bounds__(kThreads)
   pin_loads(m);
   __syncthreads();
 
-  // The W table is double-buffered: the next radius's is filled between the two
-  // barriers of a radius, beside stage B.  Blocks without the packed column
+  // The next radius's W table is filled between the two barriers of a radius, beside
+  // stage B, in a second buffer (stage A's reads of the first have ended; with one
+  // the compiler spilled 44 B and reloaded them in the loop).  Blocks without the packed column
   // take a loop without it: a branch per value made each wait for its own LDS
   // read, and the first use of the spectrum loads inside the loop waited for
   // the stores of the radius before.  1024^3 x 32: 32.2-33.1 -> 27.6-27.8 ms with
@@ -294,8 +296,9 @@ __global__ void __launch_bounds__(x2048::kThreads)
   __shared__ uint32_t bufX[N2 * CF2];
   __shared__ uint32_t bufY[N2 * CF2];
   constexpr int kWT2 = (CF2 + 1) * NF2;
-  __shared__ float wtab[2][kWT2];  // of two radii: [|fx|][column], then the kz = N/2 column
+  __shared__ float wtab[kWT2];     // [|fx|][column], then the kz = N/2 column
   extern __shared__ float4 wsh[];  // W(x) interpolation table (wM intervals)
+  static_assert((2 * N2 * CF2 + kWT2) * 4 + 16 * kWTableMax <= 160 * 1024, "LDS with the longest W(x) table");
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
@@ -334,13 +337,12 @@ __global__ void __launch_bounds__(x2048::kThreads)
     constexpr bool PK = decltype(pk)::value;
     auto fill = [&](int rl) {
       const float dkR = dk * rc[r0 + rl].R;
-      fill_wcolumns<N2, CF2, T2, PK>(wtab[rl & 1], fy2, kz0, dkR, dkR * winvh, invN3, wsh, wM, tid);
+      fill_wcolumns<N2, CF2, T2, PK>(wtab, fy2, kz0, dkR, dkR * winvh, invN3, wsh, wM, tid);
     };
     fill(0);
     __syncthreads();
 #pragma unroll 1
     for (int rl = 0; rl < nb; ++rl) {
-      const float* wt = wtab[rl & 1];
       // opaque zero: the radius-invariant LDS and store addresses and the
       // stage-C twiddles are rebuilt per radius instead of held in registers
       int zo = 0;
@@ -354,10 +356,10 @@ __global__ void __launch_bounds__(x2048::kThreads)
         for (int j = 0; j < 4; ++j) {
           const int kx = b + 128 * (4 * g + j);
           const int fa = (kx <= N2 / 2) ? kx : N2 - kx;
-          const float w0 = wt[fa * CF2 + c];
+          const float w0 = wtab[fa * CF2 + c];
           x[j] = cscale(m[4 * t + j], w0);
           if constexpr (PK) {  // every lane computes it: no branch
-            const float wn = wt[CF2 * NF2 + fa];
+            const float wn = wtab[CF2 * NF2 + fa];
             const float2 dn = DN[(long long)(kx + zo) * N2 + ky];
             const float2 s = make_float2(fmaf(w0, m[4 * t + j].x, -(wn * dn.y)), fmaf(wn, dn.x, w0 * m[4 * t + j].y));
             x[j] = make_float2(packed ? s.x : x[j].x, packed ? s.y : x[j].y);

@@ -168,6 +168,9 @@ __global__ void __launch_bounds__(kFxThreads)
   __shared__ half8_t s_gA[2][2][64];  // the 16-point DFT (stage A), [block h][hi/lo][lane]
   __shared__ float2 s_twc[3 * 256];   // exp(2 pi i m / 1024), m < 768 (stage C)
   extern __shared__ float4 wsh[];     // W(x) interpolation table (wM intervals)
+  static_assert(kN * kCF * 8 + 2 * kWT * 4 + 4 * 64 * 16 + 3 * 256 * 8 + 4 * kFxThreads / 64 + 64 +
+                        16 * kWTableSplitMax <= 160 * 1024,
+                "LDS with the longest W(x) table");
 
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63;
