@@ -208,7 +208,7 @@ hipError_t launch_moments_finish(const double2* partial, int nblk, int nrad, dou
 hipError_t launch_history(const float* zre, long long total, unsigned int* counts, double dz, int* range,
                           hipStream_t s);
 // history correction (bubble_kernels.hip)
-// scratch: N^3 floats and N + 1 doubles, 8-byte aligned
+// N a multiple of 16; scratch: N^3 floats and N + 1 doubles, 16-byte aligned
 hipError_t launch_skewers(const float* zre, const float* zcur, const SkewerParams& p, void* scratch, double* sums,
                           unsigned int* counts, int* fail, hipStream_t s);
 // rising: chist[q] <= chist[q + 1] for all q
