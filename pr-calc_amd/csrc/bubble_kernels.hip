@@ -254,7 +254,12 @@ __global__ void __launch_bounds__(256)
       out = 0.01f;
     } else {
       out = __builtin_nanf("");
-      int q0 = 0;
+      auto at = [&](int q) {
+        const float f = (x - c[q]) / (c[q + 1] - c[q]);
+        const double z0 = 49.9 + (double)((float)q * dzch);
+        const double z1 = 49.9 + (double)((float)(q + 1) * dzch);
+        return (float)((double)(1.0f - f) * z0 + (double)f * z1);
+      };
       if (rising) {
         int lo = 0, hi = kNCHistory - 1;  // chist[hi] >= x
         while (lo < hi) {
@@ -262,16 +267,14 @@ __global__ void __launch_bounds__(256)
           if (c[mid] >= x) hi = mid;
           else lo = mid + 1;
         }
-        q0 = max(hi - 1, 0);
-      }
-      for (int q = q0; q < kNCHistory - 1; ++q) {
-        if (x >= c[q] && x <= c[q + 1]) {
-          const float f = (x - c[q]) / (c[q + 1] - c[q]);
-          const double z0 = 49.9 + (double)((float)q * dzch);
-          const double z1 = 49.9 + (double)((float)(q + 1) * dzch);
-          out = (float)((double)(1.0f - f) * z0 + (double)f * z1);
-          break;
-        }
+        const int q = max(hi - 1, 0);
+        if (x >= c[q] && x <= c[q + 1]) out = at(q);
+      } else {
+        for (int q = 0; q < kNCHistory - 1; ++q)
+          if (x >= c[q] && x <= c[q + 1]) {
+            out = at(q);
+            break;
+          }
       }
     }
   }
