@@ -10,6 +10,8 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "d2z_device.h"
 #include "d2z_kernels.h"
 #include "fft_core.h"
@@ -96,8 +98,8 @@ __global__ void __launch_bounds__(256) k_take_field(const float* __restrict__ sr
 constexpr int kHistWindow = 36000;  // bins per window: 144 KB of LDS
 constexpr int kHistWindows = (kNHistory + kHistWindow - 1) / kHistWindow;
 
-__device__ __forceinline__ int history_bin(float z, double dz, double rdz) {
-  const double q = history_q(z, dz, rdz);
+__device__ __forceinline__ int history_bin(float z, double dz) {
+  const double q = ((double)z - 49.9) / dz;
   return (q > -1.0 && q < (double)kNHistory) ? (int)q : -1;  // NaN: -1
 }
 
@@ -153,7 +155,7 @@ __global__ void __launch_bounds__(1024) k_history_range(const float* __restrict_
 }
 
 __global__ void __launch_bounds__(1024) k_history(const float* __restrict__ zre, long long total,
-                                                  unsigned int* __restrict__ counts, double dz, double rdz,
+                                                  unsigned int* __restrict__ counts, double dz,
                                                   const int* __restrict__ range) {
   __shared__ unsigned int h[kHistWindow];
   if (range[1] < 0) return;  // no cell in any bin
@@ -167,15 +169,18 @@ __global__ void __launch_bounds__(1024) k_history(const float* __restrict__ zre,
   for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < n4; id += 2 * stride) {
     const float4 v = z4[id];
     const float4 u = id + stride < n4 ? z4[id + stride] : make_float4(NAN, NAN, NAN, NAN);
-    const float z[8] = {v.x, v.y, v.z, v.w, u.x, u.y, u.z, u.w};
+    // divisions, without a branch: a product by 1/dz that divides near the edges of a
+    // bin (history_q) took 1177 instead of 963 us at 1024^3, 166 instead of 136 at 512^3
+    const int b[8] = {history_bin(v.x, dz), history_bin(v.y, dz), history_bin(v.z, dz), history_bin(v.w, dz),
+                      history_bin(u.x, dz), history_bin(u.y, dz), history_bin(u.z, dz), history_bin(u.w, dz)};
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int b = history_bin(z[q], dz, rdz), r = b - lo;
-      if (b >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
+      const int r = b[q] - lo;
+      if (b[q] >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
     }
   }
   for (long long id = 4 * n4 + (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total; id += stride) {
-    const int b = history_bin(zre[id], dz, rdz), r = b - lo;
+    const int b = history_bin(zre[id], dz), r = b - lo;
     if (b >= 0 && r >= 0 && r < kHistWindow) atomicAdd(&h[r], 1u);
   }
   __syncthreads();
@@ -501,12 +506,12 @@ hipError_t launch_history(const float* zre, long long total, unsigned int* count
   if (g < 1) g = 1;
   hipLaunchKernelGGL(k_history_range, dim3((unsigned)g), dim3(1024), 0, s, zre, total, range, dz, zmin, zmax);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  // a block adds up to ~30000 bins to the global counts: give it 2^18 cells for them
-  long long gh = (total + (1 << 18) - 1) >> 18;
-  if (gh > 256) gh = 256;
-  if (gh < 1) gh = 1;
-  hipLaunchKernelGGL(k_history, dim3((unsigned)gh, kHistWindows), dim3(1024), 0, s, zre, total, counts, dz, 1.0 / dz,
-                     range);
+  // 2^13 cells a block (8 per thread), but where that is more than 128 blocks, each of
+  // which adds up to ~30000 bins to the global counts, 2^15, up to one block per CU.
+  // Blocks of 2^18 cells took 67 us at 64^3 and 128^3, 73 at 256^3, these 7, 10 and 28.
+  const long long most = std::min(256LL, std::max(128LL, total >> 15));
+  const long long gh = std::max(1LL, std::min(most, total >> 13));
+  hipLaunchKernelGGL(k_history, dim3((unsigned)gh, kHistWindows), dim3(1024), 0, s, zre, total, counts, dz, range);
   return hipGetLastError();
 }
 
