@@ -431,6 +431,10 @@ struct PkBins {  // the block's sums, in LDS
   unsigned n[kPkMaxBins];
   double p[kPkMaxBins], o[kPkMaxBins], k[kPkMaxBins];
 };
+// kx per item of the planes kz = 0 and N/2: a serial chain, which at 16 set the time of
+// the smallest grids (16^3 and 32^3 5.8 and 6.0 us, at 4 3.6 and 3.4; at 64^3 the same,
+// above it 16 is up to 6% faster with a single bin, where each item adds to it)
+__host__ __device__ constexpr int pk_plane(int N) { return N <= 64 ? 4 : 16; }
 __device__ __forceinline__ void pk_flush(PkBins& B, const PkSum& a) {
   if (a.bin < 0) return;
   atomicAdd(&B.n[a.bin], a.n);
@@ -472,9 +476,9 @@ __global__ void __launch_bounds__(256)
     a.o += (double)(1.0f / rk2);
     a.k += (double)rk;
   };
-  // items: (kz block, ky) rows of S, 256 / C threads along kx; then 16 kx of the
+  // items: (kz block, ky) rows of S, 256 / C threads along kx; then X kx of the
   // planes kz = 0 and N/2, threads along ky
-  const int nrow = (Nh / C) * N, npl = N / 16;
+  const int nrow = (Nh / C) * N, X = pk_plane(N), npl = N / X;
   for (int item = blockIdx.x; item < nrow + 2 * npl; item += gridDim.x) {
     if (item < nrow) {
       const int ky = item % N, kz = (item / N) * C + t % C;
@@ -484,13 +488,13 @@ __global__ void __launch_bounds__(256)
 #pragma unroll 4
       for (int kx = t / C; kx < N; kx += 256 / C) add(freq(kx), fy, fz, row[kx * C]);
     } else {
-      const int q = item - nrow, kz = q < npl ? 0 : Nh, x0 = (q < npl ? q : q - npl) * 16;
+      const int q = item - nrow, kz = q < npl ? 0 : Nh, x0 = (q < npl ? q : q - npl) * X;
       const float2* pl = kz == 0 ? D0 : DN;
       const float fz = freq(kz);
       for (int ky = t; ky < N; ky += 256) {
         const float fy = freq(ky);
 #pragma unroll 4
-        for (int x = 0; x < 16; ++x) add(freq(x0 + x), fy, fz, pl[(long long)(x0 + x) * N + ky]);
+        for (int x = 0; x < X; ++x) add(freq(x0 + x), fy, fz, pl[(long long)(x0 + x) * N + ky]);
       }
     }
   }
@@ -1535,7 +1539,7 @@ template <int N>
 static hipError_t pk_impl(const float2* S, const float2* D0, const float2* DN, float dk, float lnkmin, float dlnk,
                           int nk, double pscale, unsigned long long* count, double* sums, hipStream_t s) {
   // persistent: up to 8 blocks per CU, each with its own LDS sums
-  long long g = (long long)N * ((N / 2) / Blk<N>::C) + 2 * (N / 16);
+  long long g = (long long)N * ((N / 2) / Blk<N>::C) + 2 * (N / pk_plane(N));
   if (g > 2048) g = 2048;
   hipLaunchKernelGGL((k_pk<Blk<N>::C>), dim3((unsigned)g), dim3(256), 0, s, S, D0, DN, N, dk, lnkmin, dlnk, nk, pscale,
                      count, sums);
