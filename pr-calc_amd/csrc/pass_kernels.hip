@@ -538,6 +538,8 @@ struct FxLds {
   // beside the largest W(x) table and are read from memory
   static constexpr bool TW = P::L <= 1024;
   static constexpr int NTW = TW ? (plan_tw_size<P>() > 0 ? plan_tw_size<P>() : 1) : 1;
+  static constexpr size_t BYTES = sizeof(float2) * (SMEM + NTW) + sizeof(float) * WTAB;
+  static_assert(BYTES + sizeof(float4) * kWTableMax <= 160 * 1024, "LDS with the longest W(x) table");
 };
 
 // One tile (ky, kz block, column sub-tile) of the fused x pass for nb radii.
@@ -1054,8 +1056,7 @@ constexpr size_t mb_lds_n(MBPass pass) {
     case MBPass::kFwdX:
     case MBPass::kInvY: return sizeof(float2) * TilePlan<N>::L * Blk<N>::C;
     case MBPass::kFx:
-      return sizeof(float2) * (FxLds<PF, FxCols<N>::CF>::SMEM + FxLds<PF, FxCols<N>::CF>::NTW) +
-             sizeof(float) * FxLds<PF, FxCols<N>::CF>::WTAB;
+      return FxLds<PF, FxCols<N>::CF>::BYTES;
     case MBPass::kFz:
       return sizeof(float2) * (FzLds<PZ>::SMEM + FzLds<PZ>::NTW + PZ::L);
     default: return 0;
