@@ -163,7 +163,9 @@ __device__ __forceinline__ float filter_coef(int m, float dkR, float invN3) {
   return tophat(__builtin_amdgcn_sqrtf((float)m) * dkR) * invN3;
 }
 
-// The table's value for M > 0, without branches
+// W(|k| R) / N^3 for |k| = km dk from the interpolation table (M > 0 entries c0..c3,
+// one per interval of length 1/invh in x = |k| R; dkRh = dk R invh), without
+// branches; km = 0 gives 0
 __device__ __forceinline__ float interpolated_filter(float km, float dkRh, float invN3, const float4* tab, int M) {
   const float u = km * dkRh;
   int i = (int)u;
@@ -174,18 +176,8 @@ __device__ __forceinline__ float interpolated_filter(float km, float dkRh, float
   return km == 0.0f ? 0.0f : w;
 }
 
-// W(|k| R) / N^3 from the interpolation table (entries c0..c3 per interval of
-// length 1/invh in x = |k| R) for |k| = km dk; dkRh = dk R invh.  M = 0 or
-// km = 0 fall back to the exact value / the zeroed mean mode.
-__device__ __forceinline__ float filter_from_table(float km, float dkR, float dkRh, float invN3,
-                                                   const float4* tab, int M) {
-  if (km == 0.0f) return 0.0f;
-  if (M == 0) return tophat(km * dkR) * invN3;
-  return interpolated_filter(km, dkRh, invN3, tab, M);
-}
-
-// The same in two steps for tables that reuse |k| over radii:
-// kmag_grid(m) = |k| / dk, filter_of_kmag(kmag_grid(m), dkR, invN3) ==
+// filter_coef in two steps, for tables that reuse |k| over radii (and, with kmag_grid,
+// interpolated_filter): kmag_grid(m) = |k| / dk, filter_of_kmag(kmag_grid(m), dkR, invN3) ==
 // filter_coef(m, dkR, invN3) bit for bit.
 __device__ __forceinline__ float kmag_grid(int m) { return __builtin_amdgcn_sqrtf((float)m); }
 __device__ __forceinline__ float filter_of_kmag(float km, float dkR, float invN3) {
@@ -196,8 +188,8 @@ __device__ __forceinline__ float filter_of_kmag(float km, float dkR, float invN3
 // One radius's W table of a matrix x pass block (N points, CF columns from kz0 on,
 // NT threads): wt[f CF + c] = scale W at (|fx| = f, kz0 + c), f <= N/2, and, PK, the
 // kz = N/2 column behind them.  A thread keeps its column, so |k| is two integer
-// operations and a square root on the way to the table read; the values are
-// filter_from_table's bit for bit.
+// operations and a square root on the way to the table read.  M = 0: no W(x) table
+// covers the run, W is evaluated.
 template <int N, int CF, int NT, bool PK>
 __device__ __forceinline__ void fill_wcolumns(float* wt, int fy2, int kz0, float dkR, float dkRh, float scale,
                                               const float4* tab, int M, int tid) {
@@ -241,7 +233,8 @@ __host__ __device__ inline double barrier_offset(float dd, float erfizeta) {
 // q = ((double)z - 49.9) / dz, the history bin before truncation, with the same
 // integer part: a product by 1/dz (rdz) is within 3e-11 of the quotient for any
 // q of the table's range, so only values near an integer (about 2e-7 of all) take
-// the division, which costs some thirty FP64 instructions.
+// the division, which costs some thirty FP64 instructions.  For the remap, whose time
+// is its loads and stores; the histogram, many values a thread, divides.
 __device__ __forceinline__ double history_q(float z, double dz, double rdz) {
   const double d = (double)z - 49.9;
   double q = d * rdz;
