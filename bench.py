@@ -49,14 +49,28 @@ WORKLOADS = {
 MULTIBOX = [(128, 200.0), (192, 300.0), (256, 400.0)]
 MODES = {"plain": 0, "fused": 1, "mixed": 2, "half": 3}
 METRIC = "cell\u00b7radius updates/s at 1024\u00b3\u00d796R: batched mixed vs plain FP32; HBM GB/s"
-DTYPES = {"plain": "f32", "fused": "f32",
-          "mixed": "f32 transforms: radix-16 stages on f16 matrix cores with split hi/lo operands "
-                   "(hi*hi + hi*lo + lo*hi) and f32 accumulation; f32 intermediates, f32 vector stages",
-          "half": "f16 storage and f16 matrix-core radix-16 stages with f32 accumulation; f32 vector and barrier"}
 STORE_BYTES = {"plain": 4, "fused": 4, "mixed": 4, "half": 2}
 
 
 FX_MAX_RADII = 16  # radii per fused x-pass launch (the library's launch limit)
+
+
+def plan_names(plan) -> dict | None:
+    """A context's FFT plans of the x and z passes (D2Z.plan()) by name."""
+    return {a: "matrix" if plan[f"{a}_plan"] else "vector" for a in ("x", "z")} if plan else None
+
+
+def dtype_of(mode: str, plans: dict | None) -> str:
+    """The arithmetic of a mode under the FFT plans that ran (plan_names)."""
+    if mode in ("plain", "fused"):
+        return "f32"
+    on = " and ".join(a for a in ("x", "z") if plans[a] == "matrix")
+    if mode == "mixed":
+        return "f32" if not on else (
+            f"f32 transforms: radix-16 stages of {on} on f16 matrix cores with split hi/lo operands "
+            "(hi*hi + hi*lo + lo*hi) and f32 accumulation; f32 intermediates, f32 vector stages")
+    return "f16 storage, f32 transforms and barrier" if not on else (
+        f"f16 storage and f16 matrix-core radix-16 stages of {on} with f32 accumulation; f32 vector and barrier")
 
 
 def kernel_alg_bytes(name: str, N: int, nb: int, store_bytes: int) -> float:
@@ -81,16 +95,21 @@ def kernel_alg_bytes(name: str, N: int, nb: int, store_bytes: int) -> float:
     return table.get(name, 0.0) * cells
 
 
-def traffic_profile(workload: str, mode: str) -> dict:
+def traffic_profile(workload: str, mode: str, plans: dict | None = None) -> dict:
     """The committed rocprofv3 counter summary of a workload and mode
-    (FETCH_SIZE and WRITE_SIZE per launch, calibrated), or {}."""
-    f = ROOT / "profiles" / f"traffic_{workload}_{mode}.json"
-    if not f.exists():
-        return {}
-    try:
-        return json.loads(f.read_text())
-    except Exception:
-        return {}
+    (FETCH_SIZE and WRITE_SIZE per launch, calibrated), or {}.  With plans
+    (plan_names), the one of these FFT plans: other plans run other kernels."""
+    main = f"traffic_{workload}_{mode}"
+    for f in sorted((ROOT / "profiles").glob(f"{main}*.json"), key=lambda f: (f.stem != main, f.name)):
+        try:
+            prof = json.loads(f.read_text())
+        except Exception:
+            continue
+        if plans is None:
+            return prof if f.stem == main else {}
+        if prof.get("_about", {}).get("fft_plans") == plans:
+            return prof
+    return {}
 
 
 def measured_bytes(entry, alg_per_launch: float):
@@ -173,10 +192,10 @@ def main():
     ap.add_argument("--steps", type=int, default=5)
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--mode", default="mixed", choices=list(MODES),
-                    help="mixed (default): fused path whose radix-16 stages run on the matrix cores with "
-                         "split hi/lo FP16 operands and FP32 accumulation, FP32 intermediates; fused: fused "
-                         "path on the vector ALUs in FP32; half: fused path with FP16 intermediates and plain "
-                         "FP16 matrix-core stages; plain: one radius per pass in FP32")
+                    help="mixed (default): fused path with FP32 intermediates and an FP32 barrier, whose radix-16 "
+                         "stages can run on the matrix cores with split hi/lo FP16 operands and FP32 accumulation "
+                         "(--plan, or as tuned); fused: fused path on the vector ALUs in FP32; half: fused path with "
+                         "FP16 intermediates and plain FP16 matrix-core stages; plain: one radius per pass in FP32")
     ap.add_argument("--no-plain-compare", action="store_true",
                     help="skip the plain FP32, fused FP32 and half paths measured beside the default one")
     ap.add_argument("--workload", default="c3_1024", choices=list(WORKLOADS) + ["c4_multibox"])
@@ -240,6 +259,7 @@ def main():
     # request to fit the intermediates in HBM)
     nb = d.launch_config()["radii_per_launch"] if args.mode != "plain" else 1
     plan = d.plan() if args.mode != "plain" else None
+    plans = plan_names(plan)
     fx_nb = plan["x_radii_per_launch"] if plan else FX_MAX_RADII
     store = STORE_BYTES[args.mode]
 
@@ -255,7 +275,7 @@ def main():
             launches = [min(fx_nb, n - o) for n in launches for o in range(0, n, fx_nb)]
         return sum(kernel_alg_bytes(name, N, n, store) for n in launches)
 
-    tprof = traffic_profile(args.workload, args.mode)
+    tprof = traffic_profile(args.workload, args.mode, plans)
 
     def kernel_roof(name):
         """A kernel's algorithmic bytes over its event time, and its measured
@@ -330,13 +350,12 @@ def main():
         "metric": METRIC,
         "value": value, "unit": "cell*radius/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": ms_step, "higher_is_better": True,
-        "scaling": "weak", "vs_baseline": None, "dtype": DTYPES[args.mode],
+        "scaling": "weak", "vs_baseline": None, "dtype": dtype_of(args.mode, plans),
         "data": "synthetic",
         "config": {"workload": f"{N}^3 box {box:g} Mpc/h, {NS} radii 1 cell..{rmax:g} Mpc/h, "
                                f"zeta 40, Mmin 1e8 Msun/h, GRF seed 1", "mode": args.mode,
                    "radii_per_batch": nb, "x_pass_radii_per_launch": min(nb, fx_nb),
-                   "fft_plans": ({"x": ("matrix" if plan["x_plan"] else "vector"),
-                                  "z": ("matrix" if plan["z_plan"] else "vector")} if plan else None),
+                   "fft_plans": plans,
                    "autotuned": tuning is not None},
         "graph_ms_per_step": graph_ms,
         "graph_ms_per_step_median": float(np.median(step_ms)),
@@ -368,11 +387,10 @@ def path_rate(lp, mode: str, steps: int, tune: bool = True) -> dict:
         d.run_async()
     d.sync()
     el = time.perf_counter() - t0
-    plan = d.plan()
+    plans = plan_names(d.plan())
     d.close()
     return {"value": N ** 3 * NS * steps / el, "ms_per_step": el / steps * 1e3, "steps": steps,
-            "dtype": DTYPES[mode], "fft_plans": {"x": "matrix" if plan["x_plan"] else "vector",
-                                                  "z": "matrix" if plan["z_plan"] else "vector"}}
+            "dtype": dtype_of(mode, plans), "fft_plans": plans}
 
 
 def plain_fp32_rate(lp, steps: int) -> dict:
