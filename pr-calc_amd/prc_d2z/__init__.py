@@ -173,6 +173,12 @@ def _to_cparams(p: D2ZParams) -> CParams:
     return c
 
 
+def _build_id(lib) -> str:
+    """The loaded library's build: a digest of its file."""
+    import hashlib
+    return hashlib.sha256(Path(lib._name).read_bytes()).hexdigest()[:16]
+
+
 class D2Z:
     """One box on one GPU: the reference's delta2zreion operator."""
 
@@ -376,10 +382,13 @@ class D2Z:
 
     def autotune(self, cache: str | os.PathLike | None = None) -> dict:
         """Pick FFT plans and launch shape with the library's autotuner.  With
-        ``cache`` (a JSON file) a stored choice for this (device, N, mode) is
-        reused, and a new one is stored."""
+        ``cache`` (a JSON file) a stored choice for this (device, N, mode) and this
+        build of the library is reused, and a new one is stored: another build's
+        fastest plans and grids need not be this one's."""
         import json
         key = f"{self.params.device}:N{self.N}:mode{self.params.mode}"
+        if cache is not None:
+            key += f":lib{_build_id(self.lib)}"
         if cache is not None and Path(cache).exists():
             table = json.loads(Path(cache).read_text())
             if key in table:
