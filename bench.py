@@ -294,8 +294,7 @@ def main():
             "b_alg_path": B_ALG_PATH[args.mode],
             "path_achieved": value * B_ALG_PATH[args.mode] / 1e9,
             "path_frac": value * B_ALG_PATH[args.mode] / 1e9 / HBM_PEAK_GBS}
-    # every fused pass, not only the dominant one (in the mixed path the x and
-    # y passes take about the same time per step)
+    # every fused pass, not only the dominant one
     if args.mode != "plain":
         roof["fused_kernels"] = {k: kernel_roof(k) for k in ("fx_filter", "inv_y", "fz_barrier") if k in kernels}
     # measured HBM bytes of the whole step (rocprof FETCH_SIZE + WRITE_SIZE per

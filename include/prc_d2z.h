@@ -49,12 +49,13 @@ enum prc_d2z_status {
 
 /* Execution paths over the same arithmetic contract. */
 enum prc_d2z_mode {
-  PRC_D2Z_PLAIN_FP32 = 0, /* separate kernels: filter, 3 c2r passes, barrier, moments */
+  PRC_D2Z_PLAIN_FP32 = 0, /* one radius at a time: filter, 3 c2r passes, the last with barrier and sums */
   PRC_D2Z_FUSED_FP32 = 1, /* filter fused into the first inverse pass, barrier/max into the last,
                              radii_per_launch radii per launch off one resident spectrum */
-  PRC_D2Z_FUSED_MIXED = 2, /* fused; at N = 1024 the x and z passes' radix-16 stages run on the matrix
-                             cores with split hi/lo FP16 operands and FP32 accumulation (FP32-grade
-                             transforms), FP32 intermediates; other N as FUSED_FP32 */
+  PRC_D2Z_FUSED_MIXED = 2, /* fused, FP32 intermediates and an FP32 barrier; at N = 1024 the x and z passes'
+                             radix-16 stages run on the matrix cores with split hi/lo FP16 operands and
+                             FP32 accumulation (FP32-grade transforms) unless prc_d2z_set_plan or the
+                             autotuner, which finds the vector plans faster, says otherwise */
   PRC_D2Z_FUSED_HALF = 3   /* fused, with FP16 storage of the inter-pass intermediates (and, at N = 1024,
                              plain FP16 matrix-core radix-16 stages): narrower than FP32 */
 };
@@ -250,7 +251,8 @@ int prc_d2z_get_launch_config(const prc_d2z_ctx* ctx, int* radii_per_launch, int
  * 4, 8, 16 stages on the vector ALUs) or the matrix-core plans (radix-16
  * stages on the matrix cores: split hi/lo FP16 operands in the mixed mode at
  * N = 1024; plain FP16 in the half mode, x pass at N = 1024 and 2048, z pass
- * at N = 1024).  Default: matrix-core where the mode and N have them; asking
+ * at N = 1024).  A context starts with the matrix-core plans where the mode and N
+ * have them, whether or not they are the faster ones (prc_d2z_autotune); asking
  * for one that does not exist returns UNSUPPORTED_N.  x_radii_per_launch:
  * radii per x-pass launch, 1..16. */
 enum prc_d2z_plan { PRC_D2Z_PLAN_VECTOR = 0, PRC_D2Z_PLAN_MATRIX = 1 };

@@ -1,6 +1,7 @@
 // Set-up and element-wise kernels of the delta2zreion path (gfx950): twiddle
 // tables, the FP64 scalar set-up (sigma(R) quadrature, erfc^-1 root, growth
-// factors), the plain path's barrier and moments, the history histogram.
+// factors), the plain path's sigma_grid reduction, the input field, the history
+// histogram.
 //
 // Reference: c++/src/delta2zreion_d2z.C:12-38,97-146,206-216,
 // c++/src/cosmology.C:174-309, c++/src/math.C:23-61,
