@@ -101,10 +101,21 @@ __device__ __forceinline__ int walk_row(const float* __restrict__ row, long long
 // first cell below zc, at most n >= 16.  A lane walking alone waits for one load per
 // step, and its wave for the longest of 64 walks (256^3, 20000 skewers: 18.2 ms).
 // Here 16 lanes look at a walk's first 16 cells, 32 walks in flight; those that go
-// on are taken by the whole wave, 64 cells a look and kWalks walks in flight.
+// on are taken by the whole wave, 64 cells a look and kWalks walks in flight.  Rows of
+// fewer than ALONE cells are short enough for lanes alone: 16^3 x 20000 2.30 -> 2.08
+// ms, 32^3 x 16 143 -> 119 us (but 32^3 x 20000, with the copy, 1.95 -> 2.35 ms).
 constexpr int kWalks = 4;
+template <int ALONE>
 __device__ __forceinline__ int walks(const float* __restrict__ f, long long row, long long step, int c0, int n, float zc,
                                      bool on, int lane) {
+  if (n < ALONE) {
+    int k = 0, c = c0;
+    if (on) do {
+        c = c + 1 == n ? 0 : c + 1;
+        ++k;
+      } while (k < n && !(f[row + c * step] < zc));
+    return k;
+  }
   const unsigned long long todo = __ballot(on);
   const int m = (lane & 15) + 1;
   int r = 0;
@@ -201,9 +212,10 @@ __global__ void __launch_bounds__(kSkewerThreads)
     if (!found) atomicOr(fail, 1);
   }
   // +y (bubblehistory_d2z.C:159-183) and +z (:196-221): at most N steps each
-  const int my = YZ ? walks(zyz, i0 * NN + (long long)k0 * N, 1, j0, N, zc, found, lane)
-                    : walks(zre, i0 * NN + k0, N, j0, N, zc, found, lane);
-  const int mz = walks(zre, i0 * NN + (long long)j0 * N, 1, k0, N, zc, found, lane);
+  constexpr int kAlone = YZ ? 32 : 64;
+  const int my = YZ ? walks<kAlone>(zyz, i0 * NN + (long long)k0 * N, 1, j0, N, zc, found, lane)
+                    : walks<kAlone>(zre, i0 * NN + k0, N, j0, N, zc, found, lane);
+  const int mz = walks<kAlone>(zre, i0 * NN + (long long)j0 * N, 1, k0, N, zc, found, lane);
   double dsum = 0.0;
   if (found) {
     const uint4 wf = philox4x32_10(make_uint4((uint32_t)s, (uint32_t)ix, 0xffffffffu, 0u), key);

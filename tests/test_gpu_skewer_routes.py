@@ -24,7 +24,7 @@ def _box(N, mode=FUSED_FP32, nscales=6):
     return lp, d
 
 
-@pytest.mark.parametrize("N,counts", [(16, (1, 63, 64)), (64, (63, 64, 65)), (192, (1, 63, 64)), (512, (217, 218))])
+@pytest.mark.parametrize("N,counts", [(16, (1, 63, 64)), (32, (1, 63, 64)), (64, (63, 64, 65)), (192, (1, 63, 64)), (512, (217, 218))])
 def test_routes_vs_oracle(N, counts):
     lp, d = _box(N)
     with d:
